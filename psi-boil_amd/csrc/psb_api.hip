@@ -29,6 +29,7 @@
 #include "psb_fused.h"
 #include "psb_march.h"
 #include "psb_lds.h"
+#include "psb_tail.h"
 #include "psb_internal.h"
 
 // FP32 levels evaluate the stencil in flux form (set to 0 for the plain form)
@@ -973,6 +974,104 @@ void kc_r_sweep(psb_ctx *C, const Level<T> &lv, T om0, T omega, int nprev, DevSt
   launch(std::common_type<T>(), FF(), lv.mat());
 }
 
+// ---------------------------------------------------------------------------
+// the lowest levels in one workgroup (psb_tail.h)
+// ---------------------------------------------------------------------------
+// whether level l's cycle runs there: the level above the coarsest, of at
+// most one cell vector per thread (psb_tail.h has the figures on both sides).
+// Never level 0, whose last post-sweep forms the CG's rho.
+template <typename T>
+bool tail_at(const psb_ctx *C, const Hier<T> &H, int l) {
+  if (!C->tail || l < 1 || l != (int)H.L.size() - 2) return false;
+  const Level<T> &lv = H.L[l];
+  if (lv.ae || (std::is_same<T, float>::value && !lv.d)) return false;
+  return (vec_ok<T>(lv.g) ? lv.g.N / vmax<T>() : lv.g.N) <= kTailVec;
+}
+
+template <typename T, typename M, bool FLUX>
+struct Tail {
+  psb_ctx *C;
+  Level<T> &lv, &cl;
+  TailArgs<T, M> a{};
+  Tail(psb_ctx *C_, Hier<T> &H, int l, int nu1, int nu2, T omega, T cfac)
+      : C(C_), lv(H.L[l]), cl(H.L[l + 1]) {
+    a.g = lv.g;
+    a.gc = cl.g;
+    if constexpr (std::is_same<M, _Float16>::value) a.A = lv.mat16();
+    else if constexpr (FLUX) a.A = lv.matflux();
+    else a.A = lv.mat();
+    if constexpr (FLUX) a.K = lv.matflux();
+    else a.K = lv.mat();
+    a.af = lv.aflag;
+    a.afc = cl.aflag;
+    a.c = lv.c;
+    a.sI = cl.CI >> 1;
+    a.sJ = cl.CJ >> 1;
+    a.sK = cl.CK >> 1;
+    a.nu1 = nu1;
+    a.nu2 = nu2;
+    a.omega = omega;
+    a.om0 = T(omega / lv.scale);
+    a.cfac = T((double)cfac * (cl.scale / lv.scale));
+    a.kscale = T(lv.scale);
+    a.m = H.m;
+    a.G = H.G;
+    a.kc = lv.kc;
+    a.kv = lv.kv;
+    a.krt = lv.krt;
+    a.kst = lv.kst;
+  }
+  template <bool UP, bool KMID, bool KEND, bool DOWN>
+  void launch() {
+    const int nwg = DOWN ? (a.m + kTailWaves - 1) / kTailWaves : 1;
+    const size_t lds = (size_t)(a.g.N + a.m) * sizeof(T);
+    with_v<T>(a.g, [&](auto vt) {
+      constexpr int V = decltype(vt)::value;
+      hipLaunchKernelGGL((k_tail<T, V, M, FLUX, UP, KMID, KEND, DOWN>), dim3(nwg),
+                         dim3(kTailBlock), lds, C->stream, a);
+    });
+  }
+  // the descent from the first sweep in e[0]
+  void descend() {
+    a.r = lv.r;
+    a.e = lv.e[0];
+    a.eout = lv.e[1];
+    a.zout = cl.e[1];
+    launch<false, false, false, true>();
+    a.e = lv.e[1];
+    a.zin = cl.e[1];
+  }
+  T *cycle() {
+    descend();
+    a.out = lv.e[2];
+    launch<true, false, false, false>();
+    return a.out;
+  }
+  T *kstep() {  // the two Krylov steps of kstep()
+    descend();
+    a.eout = lv.e[2];
+    a.zout = cl.e[2];
+    launch<true, true, false, true>();
+    a.r = lv.krt;
+    a.e = lv.e[2];
+    a.zin = cl.e[2];
+    a.out = lv.kz;
+    launch<true, false, true, false>();
+    return a.out;
+  }
+};
+
+template <typename T>
+T *tail_cycle(psb_ctx *C, Hier<T> &H, int l, int nu1, int nu2, T omega, T cfac, bool k) {
+  auto go = [&](auto t) { return k ? t.kstep() : t.cycle(); };
+  if constexpr (std::is_same<T, float>::value) {
+    if (H.L[l].h16()) return go(Tail<T, _Float16, true>(C, H, l, nu1, nu2, omega, cfac));
+    return go(Tail<T, T, true>(C, H, l, nu1, nu2, omega, cfac));
+  } else {
+    return go(Tail<T, T, false>(C, H, l, nu1, nu2, omega, cfac));
+  }
+}
+
 // level l's correction for its right-hand side lv.r (first sweep already in
 // lv.e[0]) by two flexible-CG steps preconditioned by the cycle on l (their
 // reductions summed by the kernels that use them, no finalize launches):
@@ -985,6 +1084,7 @@ T *kstep(psb_ctx *C, Hier<T> &H, int l, DevState *st, int nu1, int nu2, T omega,
   const Grid &g = lv.g;
   if (!lv.kc || !lv.kv || !lv.kz || !lv.krt || !lv.kst)  // kcycle_buffers() was not called
     throw HipError{hipErrorInvalidValue};
+  if (tail_at(C, H, l)) return tail_cycle<T>(C, H, l, nu1, nu2, omega, cfac, true);
   const T s = T(lv.scale);
   const int nb = nblocks<T>(g);
   T *c = vcycle<T>(C, H, l, st, nu1, nu2, omega, cfac);
@@ -1045,6 +1145,8 @@ T *vcycle(psb_ctx *C, Hier<T> &H, int l, DevState *st, int nu1, int nu2, T omega
                        C->stream, H.m, H.G, lv.r, lv.e[1], st);
     return lv.e[1];
   }
+  if (!kcycle_level(C, H, l) && tail_at(C, H, l))
+    return tail_cycle<T>(C, H, l, nu1, nu2, omega, cfac, false);
   int cur = done;
   for (int s = 1 + done; s < nu1; s++) {
     jacobi<T, false>(C, lv, lv.e[cur], lv.e[(cur + 1) % 3], nullptr, nullptr, T(0), omega, st);
@@ -2540,6 +2642,7 @@ int psb_create(psb_ctx **out, const psb_layout *L) {
     // PSB_NO_LDS set: none (for comparisons); PSB_LDS_MASK="m32,m64"
     // overrides the measured defaults (bits kLdsSweep .. kLdsCgPq)
     if (std::getenv("PSB_NO_KFUSE")) C->kfuse = false;
+    if (std::getenv("PSB_NO_TAIL")) C->tail = false;
     if (std::getenv("PSB_NO_LDS")) {
       C->lds32 = C->lds64 = 0;
     } else if (const char *m = std::getenv("PSB_LDS_MASK")) {

@@ -280,6 +280,9 @@ struct psb_ctx {
   // the K-cycle's residual update fused with the next cycle's second sweep
   // (PSB_NO_KFUSE set: separate launches, for comparisons)
   bool kfuse = true;
+  // the lowest levels in one workgroup (psb_tail.h; PSB_NO_TAIL set: one
+  // launch per phase, for comparisons)
+  bool tail = true;
   // the pressure's boundary conditions for the device assembly (all Neumann,
   // value 0: walls) and the boundary source it formed (NULL: none)
   psb_bnd bnd{};
