@@ -97,10 +97,15 @@ void with_v(const Grid &g, F f) {
 
 template <int NR>
 void finalize(psb_ctx *C, int op, int nblk, DevState *st, DevState *st2 = nullptr,
-              double *out = nullptr) {
+              double *out = nullptr, const DevState *in = nullptr) {
   hipLaunchKernelGGL((k_finalize<NR>), dim3(1), dim3(kBlock), 0, C->stream, op, nblk,
-                     C->work.partial, st, st2, out);
+                     C->work.partial, in ? in : st, st, st2, out);
 }
+
+// the partials of the CG's p.q, beside those of the other reductions (at most
+// kRhoParts per block): the x/r step reads them (fold_pq) while it leaves its own
+static_assert(kRhoParts < kMaxPartials, "p.q partials follow the others");
+Work pq_work(const psb_ctx *C) { return Work{C->work.partial + (size_t)kMaxBlocks * kRhoParts}; }
 
 // Per-kernel timing of an eager solve (psb_profile_solve_device): a kernel
 // on the finest level launched inside a scope is bracketed by two HIP
@@ -173,10 +178,13 @@ void start(psb_ctx *C, const Grid &g, DMat<T> A, const T *b, const T *x, T *r, T
               nblocks<T>(g), st);
 }
 
+// the CG p/q step; its partials (as many as the return value) go to pq_work,
+// and the x/r step sums them for alpha
 template <typename T, bool SYM, bool DIAG, bool FLUX = false>
-void cg_pq(psb_ctx *C, const Grid &g, DMat<T> A, const T *rz, const T *pold, T *pnew, T *q,
-           const uint8_t *af, DevState *st) {
+int cg_pq(psb_ctx *C, const Grid &g, DMat<T> A, const T *rz, const T *pold, T *pnew, T *q,
+          const uint8_t *af, DevState *st) {
   int nb = nblocks<T>(g);
+  const Work w = pq_work(C);
   // the stored coefficient arrays, z (or r), p in; p, q out
   ProbeScope ps(C, PSB_K_CG_PQ, g, ((SYM ? 4 : 7) + 4) * sizeof(T) + (af ? 1 : 0));
   with_v<T>(g, [&](auto vt) {
@@ -186,35 +194,87 @@ void cg_pq(psb_ctx *C, const Grid &g, DMat<T> A, const T *rz, const T *pold, T *
       nb = m.nblocks;
       if (lds_use<T>(C, kLdsCgPq) && lds_ok<V>(g))
         hipLaunchKernelGGL((k_cg_pq_lds<T, V, SYM, DIAG, FLUX>), dim3(m.nblocks), dim3(kBlock),
-                           0, C->stream, g, A, rz, pold, pnew, q, af, st, C->work, m.TI,
-                           m.ntiles, T(1));
+                           0, C->stream, g, A, rz, pold, pnew, q, af, st, w, m.TI, m.ntiles,
+                           T(1));
       else
         hipLaunchKernelGGL((k_cg_pq_march<T, V, SYM, DIAG, FLUX>), dim3(m.nblocks),
-                           dim3(kBlock), 0, C->stream, g, A, rz, pold, pnew, q, af, st,
-                           C->work, m.TI, m.ntiles);
+                           dim3(kBlock), 0, C->stream, g, A, rz, pold, pnew, q, af, st, w, m.TI,
+                           m.ntiles);
       return;
     }
     hipLaunchKernelGGL((k_cg_pq<T, V, SYM, DIAG, FLUX>), dim3(nblocks<T>(g)), dim3(kBlock), 0,
-                       C->stream, g, A, rz, pold, pnew, q, af, st, C->work);
+                       C->stream, g, A, rz, pold, pnew, q, af, st, w);
   });
-  ps.end();
-  finalize<1>(C, FIN_PQ, nb, st);
+  return nb;
 }
 
 template <typename T, bool DIAG>
 void cg_xr(psb_ctx *C, const Grid &g, const T *c, const T *p, const T *q, T *x, T *r, T *e1,
-           T omega, DevState *st, int op = -1, const Metric *mt = nullptr) {
+           T omega, DevState *st, int npq, int op = -1, const Metric *mt = nullptr) {
   const Metric m = mt ? *mt : metric(C);
+  const Fold f{npq, pq_work(C).partial, nullptr};
   {
     // x, r, p, q, c in; x, r (and e1) out
     ProbeScope ps(C, PSB_K_CG_XR, g, (DIAG ? 7 : 8) * sizeof(T));
     with_v<T>(g, [&](auto vt) {
       constexpr int V = decltype(vt)::value;
       hipLaunchKernelGGL((k_cg_xr<T, V, DIAG>), dim3(nblocks<T>(g)), dim3(kBlock), 0, C->stream,
-                         g, c, m, p, q, x, r, e1, omega, st, C->work);
+                         g, c, m, p, q, x, r, e1, omega, st, C->work, f);
     });
   }
   finalize<3>(C, op >= 0 ? op : DIAG ? FIN_XR_DIAG : FIN_XR_AC, nblocks<T>(g), st);
+}
+
+// A run of `n` CG iterations with the diagonal preconditioner (cg.cpp:66-160),
+// FP64.  On grids up to kFoldCells both scalar steps are folded into the
+// streaming kernels (k_cg_pq_di, k_cg_xr_di): two launches an iteration instead
+// of four, the state handed from st to st2 and back; the last iteration's step
+// ends in st (unless `last` is false: nobody asks for it).  Measured: 64^3 6.3
+// -> 4.5 ms per 334 iterations (5.9 + 4.7 us of kernels and two nodes), 57x45x39
+// 12.7 -> 8.8 ms, two V-cycles of 96^3 12.5 -> 8.3 ms (folding up to 2^19 cells
+// only: 8.9).  The line: every block reads every partial, which at 96^3 (1728
+// blocks) brings the pair from 25 to 32 us, as much as the two launches cost; on
+// larger grids, whose kernels stream from HBM, only alpha is folded (fold_pq).
+constexpr int kFoldCells = 1 << 20;
+bool cg_di_fold(const psb_ctx *C, const Grid &g) { return C->fold && g.N <= kFoldCells; }
+// q: two arrays with the fold (z of the iteration before is read from one,
+// q[0] at the start, while A p goes to the other); n even unless it ends there
+template <bool SYM>
+void cg_di_run(psb_ctx *C, const Grid &g, DMat<double> A, double *r, double *const p[2],
+               double *const q[2], double *x, DevState *st, DevState *st2, int n,
+               const Metric *mt = nullptr, bool last = true) {
+  const int nxr = nblocks<double>(g);
+  const bool fold = cg_di_fold(C, g);
+  DevState *cur = st;
+  for (int it = 0; it < n; it++) {
+    const double *pold = p[it & 1];
+    double *pnew = p[(it & 1) ^ 1];
+    int npq = 0;
+    if (fold) {
+      DevState *nxt = cur == st ? st2 : st;
+      const Fold f{it > 0 ? nxr : 0, C->work.partial, nxt};
+      with_v<double>(g, [&](auto vt) {
+        constexpr int V = decltype(vt)::value;
+        MarchShape m{0, 0, nxr};
+        if (!(V > 1 && g.N >= kMarchMin && march_ok<V>(g, m))) m = MarchShape{0, 0, nxr};
+        npq = m.nblocks;
+        hipLaunchKernelGGL((k_cg_pq_di<V, SYM>), dim3(npq), dim3(kBlock), 0, C->stream, g, A,
+                           q[it & 1], pold, pnew, q[(it & 1) ^ 1], cur, f, pq_work(C), m.TI,
+                           m.ntiles);
+      });
+      if (it > 0) cur = nxt;
+      with_v<double>(g, [&](auto vt) {
+        constexpr int V = decltype(vt)::value;
+        hipLaunchKernelGGL((k_cg_xr_di<V>), dim3(nxr), dim3(kBlock), 0, C->stream, g, A.c,
+                           mt ? *mt : metric(C), pnew, q[(it & 1) ^ 1], x, r, cur, C->work,
+                           Fold{npq, pq_work(C).partial, nullptr});
+      });
+    } else {
+      npq = cg_pq<double, SYM, true>(C, g, A, r, pold, pnew, q[0], nullptr, cur);
+      cg_xr<double, true>(C, g, A.c, pnew, q[0], x, r, nullptr, 0.0, cur, npq, -1, mt);
+    }
+  }
+  if (fold && last) finalize<3>(C, FIN_XR_DIAG, nxr, st, nullptr, nullptr, cur);
 }
 
 // one damped Jacobi sweep on level lv (optionally with the prolongation of
@@ -1189,7 +1249,7 @@ T *vcycle(psb_ctx *C, Hier<T> &H, int l, DevState *st, int nu1, int nu2, T omega
 // (scale A16) p / scale with FP32 arithmetic; false where it does not apply
 template <typename T>
 bool cg_pq16(psb_ctx *C, const Level<T> &f, const T *z, const T *pold, T *pnew, T *q,
-             DevState *st) {
+             DevState *st, int &npq) {
   if constexpr (std::is_same<T, float>::value) {
     MarchShape m;
     if (!C->cg_half || !f.h16() || !f.d || !vec_ok<float>(f.g) || !march_ok<4>(f.g, m))
@@ -1198,9 +1258,10 @@ bool cg_pq16(psb_ctx *C, const Level<T> &f, const T *z, const T *pold, T *pnew, 
       ProbeScope ps(C, PSB_K_CG_PQ, f.g, 4 * 2 + 4 * 4 + (f.aflag ? 1 : 0));
       hipLaunchKernelGGL((k_cg_pq_march<float, 4, true, false, true, _Float16>),
                          dim3(m.nblocks), dim3(kBlock), 0, C->stream, f.g, f.mat16(), z, pold,
-                         pnew, q, f.aflag, st, C->work, m.TI, m.ntiles, (float)(1.0 / f.scale));
+                         pnew, q, f.aflag, st, pq_work(C), m.TI, m.ntiles,
+                         (float)(1.0 / f.scale));
     }
-    finalize<1>(C, FIN_PQ, m.nblocks, st);
+    npq = m.nblocks;
     return true;
   } else {
     return false;
@@ -1215,13 +1276,14 @@ void ac_iteration(psb_ctx *C, Hier<T> &H, KrylovVecs<T> &K, DevState *st, int pa
   H.qf = C->flex ? K.q : nullptr;  // q = A p of the last direction (flexible beta)
   T *z = vcycle<T>(C, H, 0, st, nu1, nu2, omega, cfac);
   T *pold = K.p[parity], *pnew = K.p[parity ^ 1];
-  if (!cg_pq16<T>(C, f, z, pold, pnew, K.q, st)) {
+  int npq = 0;
+  if (!cg_pq16<T>(C, f, z, pold, pnew, K.q, st, npq)) {
     if (f.d)
-      cg_pq<T, true, false, true>(C, f.g, f.matflux(), z, pold, pnew, K.q, f.aflag, st);
+      npq = cg_pq<T, true, false, true>(C, f.g, f.matflux(), z, pold, pnew, K.q, f.aflag, st);
     else
-      cg_pq<T, true, false>(C, f.g, f.mat(), z, pold, pnew, K.q, f.aflag, st);
+      npq = cg_pq<T, true, false>(C, f.g, f.mat(), z, pold, pnew, K.q, f.aflag, st);
   }
-  cg_xr<T, false>(C, f.g, f.c, pnew, K.q, K.x, K.r, f.e[0], T(omega / f.scale), st, xr_op);
+  cg_xr<T, false>(C, f.g, f.c, pnew, K.q, K.x, K.r, f.e[0], T(omega / f.scale), st, npq, xr_op);
 }
 
 void destroy_graph(Graph &gr) {
@@ -1402,16 +1464,15 @@ void solve_cg_diag(psb_ctx *C, double *x, const double *b, const psb_stop *p, ps
   init_state(C, C->st64, p, p->norm, p->res_rat, p->res_tol, p->max_iter);
   zero(C, K.p[0], g.N);
   zero(C, K.p[1], g.N);
-  start<double, SYM, 0>(C, g, A, b, K.x, K.r, nullptr, 0.0, C->st64);
+  const bool fold = cg_di_fold(C, g);
+  if (fold && !K.z) K.z = C->arena.alloc<double>(g.N);
+  double *const q[2] = {K.q, K.z};
+  start<double, SYM, 0>(C, g, A, b, K.x, K.r, fold ? q[0] : nullptr, 0.0, C->st64);
   HIPCHK(hipGetLastError());
   read_state(C, C->st64);
   const int chunk = chunk_of(p);
   auto body = [&]() {
-    for (int it = 0; it < chunk; it++) {
-      const int par = it & 1;
-      cg_pq<double, SYM, true>(C, g, A, K.r, K.p[par], K.p[par ^ 1], K.q, nullptr, C->st64);
-      cg_xr<double, true>(C, g, A.c, K.p[par ^ 1], K.q, K.x, K.r, nullptr, 0.0, C->st64);
-    }
+    cg_di_run<SYM>(C, g, A, K.r, K.p, q, K.x, C->st64, C->st64b, chunk);
   };
   run_graph(C, C->gr_cgdiag, chunk * 2 + (SYM ? 1 : 0), C->st64, p->max_iter, body);
   HIPCHK(hipMemcpyAsync(x, K.x, (size_t)g.N * 8, hipMemcpyDeviceToDevice, C->stream));
@@ -1433,7 +1494,7 @@ void solve_cg_diag(psb_ctx *C, double *x, const double *b, const psb_stop *p, ps
 // previous call's contents.
 // ---------------------------------------------------------------------------
 constexpr size_t kStaticMaxCells = (size_t)1 << 21;  // 128^3 cells
-constexpr size_t kStaticStateDoubles = (sizeof(DevState) + 255) / 256 * 32;
+constexpr size_t kStaticStateDoubles = (2 * sizeof(DevState) + 255) / 256 * 32;  // two states
 constexpr size_t kStaticPartialDoubles = (size_t)kMaxBlocks * kMaxPartials;
 constexpr size_t kStaticDoubles =
     kStaticStateDoubles + kStaticPartialDoubles + 4 * kStaticMaxCells;  // 64.1 MiB
@@ -1470,8 +1531,12 @@ void solve_cg_diag_static(psb_ctx *C, double *x, const double *b, const psb_stop
   DevState *st = reinterpret_cast<DevState *>(base);
   double *partial = base + kStaticStateDoubles;
   double *r = partial + kStaticPartialDoubles;
-  double *pv[2] = {r + kStaticMaxCells, r + 2 * kStaticMaxCells};
-  double *q = r + 3 * kStaticMaxCells;
+  // four vectors, five with the fold, whose grids are a quarter of the largest
+  static_assert(5 * ((size_t)kFoldCells + 32) <= 4 * kStaticMaxCells, "");
+  const bool fold = cg_di_fold(C, g);
+  const size_t stride = fold ? ((size_t)g.N + 31) / 32 * 32 : kStaticMaxCells;
+  double *pv[2] = {r + stride, r + 2 * stride};
+  double *q[2] = {r + 3 * stride, r + (fold ? 4 : 3) * stride};
   // the launch helpers take the reduction partials from C->work
   struct WorkSwap {
     psb_ctx *C;
@@ -1483,17 +1548,13 @@ void solve_cg_diag_static(psb_ctx *C, double *x, const double *b, const psb_stop
   init_state(C, st, p, p->norm, p->res_rat, p->res_tol, p->max_iter, false);
   zero(C, pv[0], g.N);
   zero(C, pv[1], g.N);
-  start<double, SYM, 0>(C, g, A, b, x, r, nullptr, 0.0, st);
+  start<double, SYM, 0>(C, g, A, b, x, r, fold ? q[0] : nullptr, 0.0, st);
   HIPCHK(hipGetLastError());
   read_state(C, st);
   const int chunk = chunk_of(p);
   long long rounds = 0;
   while (!C->hst->done) {
-    for (int it = 0; it < chunk; it++) {
-      const int par = it & 1;
-      cg_pq<double, SYM, true>(C, g, A, r, pv[par], pv[par ^ 1], q, nullptr, st);
-      cg_xr<double, true>(C, g, A.c, pv[par ^ 1], q, x, r, nullptr, 0.0, st);
-    }
+    cg_di_run<SYM>(C, g, A, r, pv, q, x, st, st + 1, chunk);
     HIPCHK(hipGetLastError());
     read_state(C, st);
     if (++rounds > (long long)p->max_iter + 2) break;
@@ -1546,8 +1607,9 @@ void solve_cg_sgs(psb_ctx *C, double *x, const double *b, const psb_stop *p, psb
       const int par = it & 1;
       rbsgs<SYM>(C, g, A, K.z, K.r, 1, false, C->st64);
       rbsgs<SYM>(C, g, A, K.z, K.r, 0, true, C->st64);
-      cg_pq<double, SYM, false>(C, g, A, K.z, K.p[par], K.p[par ^ 1], K.q, nullptr, C->st64);
-      cg_xr<double, false>(C, g, A.c, K.p[par ^ 1], K.q, K.x, K.r, K.z, 1.0, C->st64);
+      const int npq =
+          cg_pq<double, SYM, false>(C, g, A, K.z, K.p[par], K.p[par ^ 1], K.q, nullptr, C->st64);
+      cg_xr<double, false>(C, g, A.c, K.p[par ^ 1], K.q, K.x, K.r, K.z, 1.0, C->st64, npq);
     }
   };
   run_graph(C, C->gr_cgsgs, chunk * 2 + (SYM ? 1 : 0), C->st64, p->max_iter, body);
@@ -2039,7 +2101,7 @@ void build_ref(psb_ctx *C) {
   if (nl < 2) throw std::invalid_argument("grid too small for the AC cycle");
   H.L.assign(nl, Level<double>());
   H.M.assign(nl, Metric{nullptr, nullptr, nullptr});
-  H.K.assign(nl, std::vector<double *>(4, nullptr));
+  H.K.assign(nl, std::vector<double *>(5, nullptr));
   std::vector<double> hx = C->gdx, hy = C->gdy, hz = C->gdz;
   if (hx.empty()) {
     hx.assign(C->g.nx, 1.0);
@@ -2093,7 +2155,7 @@ void build_ref(psb_ctx *C) {
     lv.r = C->harena.alloc<double>(N);     // f of this level
     lv.e[0] = C->harena.alloc<double>(N);  // phi
     if (l == 0) lv.e[1] = C->harena.alloc<double>(N);  // phi of the previous cycle
-    for (int q = 0; q < 4; q++) H.K[l][q] = C->harena.alloc<double>(N);
+    for (int q = 0; q < 5; q++) H.K[l][q] = C->harena.alloc<double>(N);
   }
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(stream));
@@ -2104,7 +2166,7 @@ void build_ref(psb_ctx *C) {
 // (call_smoother / call_solver): phi is improved in place
 template <bool SYM>
 void ref_cg(psb_ctx *C, int l, int maxit, double res_rat, double res_tol, double scale,
-            int stalecount) {
+            int stalecount, bool verdict) {
   RefHier &H = C->href;
   const Level<double> &lv = H.L[l];
   const Grid &g = lv.g;
@@ -2114,12 +2176,10 @@ void ref_cg(psb_ctx *C, int l, int maxit, double res_rat, double res_tol, double
                      scale, (double)g.N, stalecount);
   zero(C, p0, g.N);
   zero(C, p1, g.N);
-  start<double, SYM, 0>(C, g, lv.mat(), lv.r, lv.e[0], r, nullptr, 0.0, st, &H.M[l]);
-  for (int it = 0; it < maxit; it++) {
-    double *pold = (it & 1) ? p1 : p0, *pnew = (it & 1) ? p0 : p1;
-    cg_pq<double, SYM, true>(C, g, lv.mat(), r, pold, pnew, q, nullptr, st);
-    cg_xr<double, true>(C, g, lv.c, pnew, q, lv.e[0], r, nullptr, 0.0, st, -1, &H.M[l]);
-  }
+  double *const p[2] = {p0, p1}, *const qz[2] = {q, H.K[l][4]};
+  start<double, SYM, 0>(C, g, lv.mat(), lv.r, lv.e[0], r, cg_di_fold(C, g) ? q : nullptr, 0.0, st,
+                        &H.M[l]);
+  cg_di_run<SYM>(C, g, lv.mat(), r, p, qz, lv.e[0], st, C->st64b, maxit, &H.M[l], verdict);
 }
 
 // Linear::solve of one level by BiCGS with the diagonal preconditioner
@@ -2127,7 +2187,7 @@ void ref_cg(psb_ctx *C, int l, int maxit, double res_rat, double res_tol, double
 // equation's own Krylov solver (additive_cycle_functions.cpp:89-107), which
 // for the non-symmetric equations is BiCGS.  The kernels and scalar steps
 // of the single-level BiCGS solve (solve_bicgs_diag) on the level's arrays;
-// phi is improved in place.  Work vectors: the CG's four and four more
+// phi is improved in place.  Work vectors: the CG's five and three more
 // (ref_bicgs_buffers, before any capture).
 void ref_bicgs_buffers(psb_ctx *C) {
   RefHier &H = C->href;
@@ -2180,15 +2240,16 @@ struct RefPar {
   int solver;
 };
 
+// (verdict: the caller reads from the state whether the solve converged)
 void ref_solve(psb_ctx *C, int l, int maxit, double rr, double rt, double scale, int stale,
-               const RefPar &q) {
+               const RefPar &q, bool verdict = false) {
   // levels of a non-symmetric matrix hold 7 arrays (build_ref)
   if (q.solver == PSB_BICGS) {
     if (C->sym) ref_bicgs<true>(C, l, maxit, rr, rt, scale, stale);
     else ref_bicgs<false>(C, l, maxit, rr, rt, scale, stale);
   } else {
-    if (C->sym) ref_cg<true>(C, l, maxit, rr, rt, scale, stale);
-    else ref_cg<false>(C, l, maxit, rr, rt, scale, stale);
+    if (C->sym) ref_cg<true>(C, l, maxit, rr, rt, scale, stale, verdict);
+    else ref_cg<false>(C, l, maxit, rr, rt, scale, stale, verdict);
   }
 }
 
@@ -2268,7 +2329,7 @@ bool ref_flex(psb_ctx *C, const RefPar &q, int max_visits) {
   for (int v = 0; v < max_visits; v++) {
     if (l != nl - 1) {
       const int s = up ? 2 : 0;
-      ref_solve(C, l, q.mv[s], q.rr, q.rt, q.scale, q.ms[s], q);
+      ref_solve(C, l, q.mv[s], q.rr, q.rt, q.scale, q.ms[s], q, true);
       read_state(C, C->st64);
       if (C->hst->converged) {
         if (l == 0) return true;
@@ -2628,6 +2689,7 @@ int psb_create(psb_ctx **out, const psb_layout *L) {
     // hipMemset of x, say) completes before the context's kernels read it
     HIPCHK(hipStreamCreateWithFlags(&C->stream, hipStreamDefault));
     C->st64 = C->base.alloc<DevState>(1);
+    C->st64b = C->base.alloc<DevState>(1);
     C->st32 = C->base.alloc<DevState>(1);
     HIPCHK(hipHostMalloc((void **)&C->hst, sizeof(DevState), hipHostMallocDefault));
     std::memset(C->hst, 0, sizeof(DevState));
@@ -2643,6 +2705,7 @@ int psb_create(psb_ctx **out, const psb_layout *L) {
     // overrides the measured defaults (bits kLdsSweep .. kLdsCgPq)
     if (std::getenv("PSB_NO_KFUSE")) C->kfuse = false;
     if (std::getenv("PSB_NO_TAIL")) C->tail = false;
+    if (std::getenv("PSB_NO_FOLD")) C->fold = false;
     if (std::getenv("PSB_NO_LDS")) {
       C->lds32 = C->lds64 = 0;
     } else if (const char *m = std::getenv("PSB_LDS_MASK")) {
@@ -3258,7 +3321,7 @@ int psb_time_kernel(psb_ctx *C, int kernel, int reps, double *avg_ms, double *by
       f = [=]() {
         hipLaunchKernelGGL((k_cg_xr<float, 4, false>), dim3(nblocks<float>(g)), dim3(kBlock), 0,
                            stream, g, lv.c, mt, K.p[0], K.q, K.x, K.r, lv.e[0], 0.9f, C->st32,
-                           C->work);
+                           C->work, Fold{});
       };
       *bytes = N * 8 * 4;
     } else if (kernel == 3) {

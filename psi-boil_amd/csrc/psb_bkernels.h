@@ -190,7 +190,10 @@ __global__ __launch_bounds__(kBlock) void kb_cg_xr(const BSeg *segs, const uint1
   if (F.st->done) return;
   const BLev<float> &L = lev0[sg_.sys];
   cg_xr_body<float, V, false>(sp, F.g, L.c, F.met, F.p[par ^ 1], F.q, F.d, F.r, L.e[0], omega,
-                              F.st, w);
+                              F.st, w, [&](double &al) {
+                                al = F.st->alpha;
+                                return true;
+                              });
 }
 
 // reliable update: x += d (gated on a pending update unless starting)

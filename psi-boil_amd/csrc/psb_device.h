@@ -115,6 +115,9 @@ struct DevState {
   double rl2_true, bsq;                        // its L2 norm; ||b||^2 (reliable updates)
 };
 
+static_assert(sizeof(DevState) % 8 == 0, "the state is copied in 8-byte words");
+constexpr int kStateWords = (int)(sizeof(DevState) / 8);
+
 // Whether a kernel of the preconditioner on a level of n cells returns at
 // once because the solve has stopped.  Below kDoneCheckMin cells it never
 // reads the flag: the load is one more round trip to memory before the
@@ -132,10 +135,34 @@ __device__ __forceinline__ bool skip_done(const DevState *st, int n) {
 // partials in a fixed order.  Two passes avoid the device-scope fence a
 // last-block-done scheme needs, which on MI355X writes back the XCD's L2.
 // ---------------------------------------------------------------------------
+// The butterfly v += v[lane ^ o], o = 32 .. 1, without the LDS: the two half
+// waves and the halves of each swapped (permlane), then rotations within a row
+// of 16 lanes -- after the step with o = 8 lanes 8 apart hold the same value,
+// so a rotation by 4 brings lane ^ 4's -- and quad permutations.  The same
+// sums as with __shfl_xor, each step a few cycles instead of a round trip
+// through the LDS (six of them one after another in every reduction).
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return v + __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  uint64_t b = __builtin_bit_cast(uint64_t, v);
+  auto l = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+  auto h = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+  v = __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) +
+      __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+  b = __builtin_bit_cast(uint64_t, v);
+  l = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+  h = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+  v = __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) +
+      __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+  v = dpp_add<0x128>(v);  // row_ror:8
+  v = dpp_add<0x124>(v);  // row_ror:4
+  v = dpp_add<0x4e>(v);   // quad_perm [2, 3, 0, 1]
+  return dpp_add<0xb1>(v);  // quad_perm [1, 0, 3, 2]
 }
 
 template <int NR>

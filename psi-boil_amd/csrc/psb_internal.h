@@ -189,7 +189,7 @@ constexpr size_t kGraphCacheMax = 12;
 
 // the reference's AC cycle: its own levels (smallest-prime-factor
 // coarsening), each with phi (e[0]), the right-hand side f (r) and the
-// work vectors of that level's CG (r, p0, p1, q); level 0's e[1] holds the
+// work vectors of that level's CG (r, p0, p1, q, z); level 0's e[1] holds the
 // previous cycle's phi for the divergence restore
 struct RefHier {
   std::vector<Level<double>> L;
@@ -232,6 +232,7 @@ struct psb_ctx {
   double *dxc = nullptr, *dyc = nullptr, *dzc = nullptr;
   // solver state
   DevState *st64 = nullptr, *st32 = nullptr;
+  DevState *st64b = nullptr;  // the other end of st64 where a kernel folds the scalar step
   DevState *hst = nullptr;  // pinned host mirror
   double *hist = nullptr;
   int hist_cap = 0;
@@ -283,6 +284,9 @@ struct psb_ctx {
   // the lowest levels in one workgroup (psb_tail.h; PSB_NO_TAIL set: one
   // launch per phase, for comparisons)
   bool tail = true;
+  // CG-di's stop test and beta in the p/q step on small grids (PSB_NO_FOLD
+  // set: a launch of their own, for comparisons)
+  bool fold = true;
   // the pressure's boundary conditions for the device assembly (all Neumann,
   // value 0: walls) and the boundary source it formed (NULL: none)
   psb_bnd bnd{};

@@ -53,6 +53,411 @@ struct Work {
 #define PSB_TILE_END }
 
 // ---------------------------------------------------------------------------
+// pass 2 of the reductions: the partials of the kernel before it summed in a
+// fixed order and the scalar step applied, by one block (k_finalize) or by
+// every block of the kernel that needs the result (fold_step, fold_pq)
+// ---------------------------------------------------------------------------
+enum FinOp {
+  FIN_START_DIAG, FIN_START_AC, FIN_START_BICGS, FIN_PQ, FIN_XR_DIAG, FIN_XR_AC, FIN_RHO,
+  FIN_XR_RU, FIN_IR_RESID, FIN_CENTER, FIN_RELRES, FIN_BI1, FIN_BI2, FIN_BI3, FIN_RU_START,
+  FIN_RU, FIN_RU_END, FIN_ACMEAN, FIN_ACRES, FIN_RHO_FLEX
+};
+
+// what the stop tests after an iteration read of the state
+struct StopIn {
+  double res0, res_rat, res_tol, scale, ntot, rho;
+  int mini, maxit, stalecount, norm, iter, done;
+  __device__ __forceinline__ StopIn(const DevState *st)
+      : res0(st->res0), res_rat(st->res_rat), res_tol(st->res_tol), scale(st->scale),
+        ntot(st->ntot), rho(st->rho), mini(st->mini), maxit(st->maxit),
+        stalecount(st->stalecount), norm(st->norm), iter(st->iter), done(st->done) {}
+};
+struct StopOut {
+  int done, conv, reason, report;  // report < 0: report_iters stays
+};
+
+// stop logic shared by the Krylov loops (cg.cpp:121-160, bicgs.cpp:174-210),
+// after iteration s.iter with the new residual; stale: the last residuals
+__device__ inline StopOut krylov_decide(const StopIn &s, const double *stale, double res,
+                                        bool small_omega) {
+  const int i = s.iter;
+  StopOut o{0, 0, 0, -1};
+  if (!(res == res) || res > 1e300) {
+    o.done = 1; o.reason = 8;
+  } else if (res < s.res_tol && i >= s.mini - 1) {
+    o.done = 1; o.conv = 1; o.reason = 1;
+  } else if (res < s.res0 * s.res_rat && i >= s.mini - 1) {
+    o.done = 1; o.conv = 1; o.reason = 2;
+  } else if (small_omega) {
+    o.done = 1; o.reason = 6;
+  } else if (s.stalecount > 0) {
+    bool none = true;
+    for (int q = 0; q < s.stalecount; q++)
+      if (res < stale[q]) { none = false; break; }
+    if (none) { o.done = 1; o.reason = 3; }
+  }
+  if (o.done) {
+    o.report = i + 1;
+  } else if (i + 1 >= s.maxit) {
+    o.done = 1;
+    o.report = s.maxit + 1;
+  }
+  return o;
+}
+
+// the state after that decision
+__device__ inline void krylov_put(DevState *st, const StopIn &s, const StopOut &o, double res) {
+  const int i = s.iter;
+  st->res = res;
+  if (st->hist && i + 1 < st->hist_cap) st->hist[i + 1] = res;
+  if (s.stalecount > 0 && o.reason == 0) {  // the window moves on
+    for (int q = 0; q + 1 < s.stalecount; q++) st->stale[q] = st->stale[q + 1];
+    st->stale[s.stalecount - 1] = res;
+  }
+  if (o.report >= 0) st->report_iters = o.report;
+  st->converged = o.conv;
+  st->reason = o.reason;
+  st->iter = i + 1;
+  st->done = o.done;
+}
+
+__device__ inline void krylov_stop(DevState *st, double res, bool small_omega) {
+  const StopIn s(st);
+  krylov_put(st, s, krylov_decide(s, st->stale, res, small_omega), res);
+}
+
+template <class S>
+__device__ inline double ref_norm(const S *st, double sum_voldiv) {
+  // sqrt(dot_voldiv_avg)/scale with dot_voldiv_avg = d/ntot/ntot
+  // (scalar.h:317-326, cg.cpp:121)
+  double d = sum_voldiv / st->ntot;
+  d = d / st->ntot;
+  return sqrt(d) / st->scale;
+}
+
+__device__ inline void krylov_init(DevState *st, double res, double rsq, double rho) {
+  st->res0 = res;
+  st->res = res;
+  st->rsq0 = rsq;
+  st->rsq = rsq;
+  st->rho = rho;
+  st->beta = 0.0;
+  st->zmean = 0.0;
+  st->iter = 0;
+  st->report_iters = 0;
+  st->converged = 0;
+  st->reason = 0;
+  st->done = 0;
+  if (st->hist && st->hist_cap > 0) st->hist[0] = res;
+  for (int q = 0; q < st->stalecount && q < kStaleMax; q++) st->stale[q] = 1.0e24;
+  if (st->stalecount > 0) st->stale[st->stalecount - 1] = res;
+}
+
+// steps of a finished loop (or a refresh not pending) do nothing
+__device__ inline bool fin_skip(int op, const DevState *st) {
+  switch (op) {
+    case FIN_PQ: case FIN_XR_DIAG: case FIN_XR_AC: case FIN_RHO: case FIN_RHO_FLEX:
+    case FIN_XR_RU:
+    case FIN_BI1: case FIN_BI2: case FIN_BI3:
+      return st->done != 0;
+    case FIN_RU:
+      return st->done || !st->update;
+    default:
+      return false;
+  }
+}
+
+// sum of the partials of blocks [b0, b0 + nblk) in a fixed order (all
+// threads of the block receive the totals).  Four rows of 256 partials are
+// loaded together (past the end the last one, replaced by 0), so that a long
+// list costs a few round trips to memory and not one per row.
+template <int NR, int ROWS>
+__device__ __forceinline__ void fin_rows(int b0, int nblk, const double *partial,
+                                         double (&acc)[NR]) {
+  for (int q0 = threadIdx.x; q0 < nblk; q0 += ROWS * kBlock) {
+    double v[ROWS][NR];
+#pragma unroll
+    for (int h = 0; h < ROWS; h++)
+#pragma unroll
+      for (int r = 0; r < NR; r++)
+        v[h][r] = partial[(size_t)(b0 + min(q0 + h * kBlock, nblk - 1)) * NR + r];
+#pragma unroll
+    for (int h = 0; h < ROWS; h++)
+#pragma unroll
+      for (int r = 0; r < NR; r++) acc[r] += q0 + h * kBlock < nblk ? v[h][r] : 0.0;
+  }
+}
+template <int NR>
+__device__ inline void fin_sum(int b0, int nblk, const double *partial, double (&acc)[NR]) {
+  __shared__ double sm[kWaves][NR];
+#pragma unroll
+  for (int r = 0; r < NR; r++) acc[r] = 0.0;
+  if (nblk <= kBlock) fin_rows<NR, 1>(b0, nblk, partial, acc);
+  else if (nblk <= 2 * kBlock) fin_rows<NR, 2>(b0, nblk, partial, acc);
+  else fin_rows<NR, 4>(b0, nblk, partial, acc);
+  block_sum<NR>(acc, sm);
+}
+
+// the scalar step of op on the totals (one thread)
+__device__ inline void fin_apply(int op, const double *tot, DevState *st, DevState *st2,
+                                 double *out) {
+  switch (op) {
+    case FIN_START_DIAG:
+    case FIN_START_AC:
+    case FIN_START_BICGS: {
+      const double res = st->norm == 0 ? ref_norm(st, tot[0]) : sqrt(tot[1]);
+      krylov_init(st, res, tot[1], tot[2]);
+      if (res < st->res_tol) {  // cg.cpp:64, bicgs.cpp:70 early return
+        st->done = 1;
+        st->converged = 1;
+        st->reason = 7;
+      }
+      if (!(res == res)) {
+        st->done = 1;
+        st->reason = 8;
+      }
+      if (op == FIN_START_BICGS && !st->done && sqrt(fabs(tot[2])) < st->res_tol) {
+        st->done = 1;  // bicgs.cpp:89 at i = 0
+        st->reason = 4;
+        st->report_iters = 1;
+      }
+      break;
+    }
+    case FIN_PQ:
+      st->pq = tot[0];
+      st->alpha = st->rho / tot[0];  // cg.cpp:107-108
+      break;
+    case FIN_XR_DIAG:
+    case FIN_XR_AC: {
+      const double res = st->norm == 0 ? ref_norm(st, tot[0]) : sqrt(tot[1]);
+      st->rsq = tot[1];
+      krylov_stop(st, res, false);
+      if (op == FIN_XR_DIAG && !st->done) {
+        st->beta = tot[2] / st->rho;  // cg.cpp:93
+        st->rho = tot[2];
+      }
+      break;
+    }
+    case FIN_XR_RU: {  // FP32 step inside the refinement: refresh or stop
+      const double res = sqrt(tot[1]);
+      const int i = st->iter;
+      st->rsq = tot[1];
+      st->res = res;
+      st->iter = i + 1;
+      if (!(res == res) || res > 1e300) {
+        st->done = 1;
+        st->reason = 8;
+        st->report_iters = i + 1;
+      } else if (res < st->rlast * st->delta || res < sqrt(st->rsq0) * st->res_rat) {
+        st->update = 1;
+      } else if (i + 1 >= st->maxit) {
+        st->done = 1;
+        st->report_iters = st->maxit + 1;
+      }
+      break;
+    }
+    case FIN_RU_START:
+    case FIN_RU: {  // true residual after a refresh (or at the start)
+      const double rl2 = sqrt(tot[0]);
+      const double res = st->norm == 0 ? ref_norm(st, tot[1]) : rl2;
+      if (op == FIN_RU_START) {
+        krylov_init(st, res, tot[0], 0.0);
+        st->outer = 0;
+      } else {
+        st->outer += 1;
+        if (st->hist && st->outer < st->hist_cap) st->hist[st->outer] = res;
+      }
+      st->res_true = res;
+      st->rl2_true = rl2;
+      if (op == FIN_RU_START) st->bsq = tot[3];
+      st->rlast = rl2;
+      st->update = 0;
+      st->res = sqrt(tot[2]);
+      if (!(res == res)) {
+        st->done = 1;
+        st->reason = 8;
+      } else if (res < st->res_tol || res < st->res0 * st->res_rat || st->res0 == 0.0) {
+        st->done = 1;
+        st->converged = 1;
+        st->reason = 2;
+        st->report_iters = st->iter;
+      } else if (st->iter >= st->maxit) {
+        st->done = 1;
+        st->report_iters = st->maxit + 1;
+      }
+      break;
+    }
+    case FIN_ACMEAN:  // mean of the restricted right-hand side over active cells
+      st->mean[0] = tot[1] > 0.0 ? tot[0] / tot[1] : 0.0;
+      break;
+    case FIN_ACRES: {  // AC::residual: sqrt(dot_voldiv_avg(r, r)) * dt (scale = dt)
+      double d = tot[0] / st->ntot;
+      d = d / st->ntot;
+      out[0] = sqrt(d) * st->scale;
+      break;
+    }
+    case FIN_RU_END:  // true residual at exit without convergence
+      st->res_true = st->norm == 0 ? ref_norm(st, tot[1]) : sqrt(tot[0]);
+      st->rl2_true = sqrt(tot[0]);
+      break;
+    case FIN_RHO:
+    case FIN_RHO_FLEX: {
+      const double m = !st->keepmean && tot[3] > 0.0 ? tot[1] / tot[3] : 0.0;
+      const double rho = tot[0] - m * tot[2];
+      st->zmean = m;
+      if (st->iter == 0) {
+        st->beta = 0.0;
+      } else if (op == FIN_RHO) {
+        st->beta = rho / st->rho;  // Fletcher-Reeves, cg.cpp:93
+      } else {
+        // flexible: beta = -z'.A p / p.A p with z' = z - m on the active
+        // cells, so the new direction is A-orthogonal to the last one
+        // whatever the preconditioner did (Notay, SISC 22 (2000) 1444-1460)
+        const double zq = tot[4] - m * tot[5];
+        st->beta = st->pq != 0.0 ? -zq / st->pq : 0.0;
+      }
+      st->rho = rho;
+      break;
+    }
+    case FIN_IR_RESID:  // st: FP64 outer state, st2: FP32 inner state
+      st->rsq = tot[0];
+      st->res = st->norm == 0 ? ref_norm(st, tot[1]) : sqrt(tot[0]);
+      st2->mean[0] = !st2->keepmean && tot[3] > 0.0 ? tot[2] / tot[3] : 0.0;
+      break;
+    case FIN_CENTER: {
+      krylov_init(st, sqrt(tot[0]), tot[0], 0.0);
+      if (tot[0] == 0.0) st->done = 1;
+      break;
+    }
+    case FIN_RELRES:
+      out[0] = tot[0];
+      out[1] = tot[1];
+      break;
+    case FIN_BI1:
+      st->rv = tot[0];
+      st->alpha = st->rho / tot[0];  // bicgs.cpp:122-123
+      break;
+    case FIN_BI2:
+      st->rv_ss = tot[0];
+      st->rv_ts = tot[1];
+      st->rv_tt = tot[2];
+      st->omega = tot[1] / tot[2];  // bicgs.cpp:155-157
+      break;
+    case FIN_BI3: {
+      if (sqrt(st->rv_ss) < st->res_tol) {  // bicgs.cpp:134-138
+        st->done = 1;
+        st->converged = 0;
+        st->reason = 5;
+        st->report_iters = st->iter + 1;
+        break;
+      }
+      const double res = st->norm == 0 ? ref_norm(st, tot[0]) : sqrt(tot[1]);
+      st->rsq = tot[1];
+      const bool small_om = st->omega >= -st->res_tol && st->omega <= st->res_tol;
+      krylov_stop(st, res, small_om);
+      if (!st->done) {
+        // top of the next iteration: rho = r~.r, breakdown test (bicgs.cpp:84-89)
+        const double rho = tot[2];
+        if (sqrt(fabs(rho)) < st->res_tol) {
+          st->done = 1;
+          st->reason = 4;
+          st->report_iters = st->iter + 1;
+        } else {
+          st->beta = (rho / st->rho) * (st->alpha / st->omega);  // bicgs.cpp:102
+          st->rho = rho;
+        }
+      }
+      break;
+    }
+  }
+}
+
+// the scalar step of op on a copy of the state in LDS, which the whole
+// block loads at once beside the partials (the step reads a dozen fields in
+// turn: a round trip to memory each if they were read where they lie).  On
+// return S is in, changed by the step.
+template <int NR>
+__device__ inline void lds_step(int op, int nblk, const double *partial, const DevState *in,
+                                DevState &S, bool record, DevState *st2 = nullptr,
+                                double *out = nullptr) {
+  uint64_t *const sw = reinterpret_cast<uint64_t *>(&S);
+  for (int q = threadIdx.x; q < kStateWords; q += kBlock)
+    sw[q] = reinterpret_cast<const uint64_t *>(in)[q];
+  double tot[NR];
+  fin_sum<NR>(0, nblk, partial, tot);  // its barriers cover S too
+  if (threadIdx.x == 0 && !fin_skip(op, &S)) {
+    double *const hist = S.hist;
+    if (!record) S.hist = nullptr;
+    fin_apply(op, tot, &S, st2, out);
+    S.hist = hist;
+  }
+  __syncthreads();
+}
+
+__device__ inline void put_state(const DevState &S, DevState *out) {
+  const uint64_t *const sw = reinterpret_cast<const uint64_t *>(&S);
+  for (int q = threadIdx.x; q < kStateWords; q += kBlock)
+    reinterpret_cast<uint64_t *>(out)[q] = sw[q];
+}
+
+// one block: st = in after the step (in may be st)
+template <int NR>
+__global__ __launch_bounds__(kBlock) void k_finalize(int op, int nblk, const double *partial,
+                                                     const DevState *in, DevState *st,
+                                                     DevState *st2, double *out) {
+  __shared__ DevState S;
+  lds_step<NR>(op, nblk, partial, in, S, true, st2, out);
+  put_state(S, st);
+}
+
+// The step in the kernel that uses its result, instead of a one-block launch
+// between the two (4 us with its graph node on small grids, where the streaming
+// kernels take 5): every block sums the partials and takes the step.
+struct Fold {
+  int nprev = 0;  // partials of the kernel before (0: no step, its result is in the state)
+  const double *prev = nullptr;
+  DevState *out = nullptr;
+};
+
+// FIN_XR_DIAG (s: the state's fields, loaded early): returns whether the
+// solve has stopped, else beta.  Block 0 leaves the new state in out, which is
+// not in: blocks that start later still read in.
+__device__ inline bool fold_xr_diag(const Fold &f, const StopIn &s, const DevState *in,
+                                    double &beta) {
+  if (blockIdx.x == 0)
+    for (int q = threadIdx.x; q < kStateWords; q += kBlock)
+      reinterpret_cast<uint64_t *>(f.out)[q] = reinterpret_cast<const uint64_t *>(in)[q];
+  double tot[3];
+  fin_sum<3>(0, f.nprev, f.prev, tot);  // its barriers order the copy before the step's fields
+  if (s.done) return true;
+  const double res = s.norm == 0 ? ref_norm(&s, tot[0]) : sqrt(tot[1]);
+  const StopOut o = krylov_decide(s, in->stale, res, false);
+  beta = tot[2] / s.rho;  // cg.cpp:93
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    f.out->rsq = tot[1];
+    krylov_put(f.out, s, o, res);
+    if (!o.done) {
+      f.out->beta = beta;
+      f.out->rho = tot[2];
+    }
+  }
+  return o.done != 0;
+}
+
+// FIN_PQ in the kernel that takes alpha (pq and alpha are read by later
+// kernels only)
+__device__ inline double fold_pq(const Fold &f, DevState *st, double rho) {
+  double tot[1];
+  fin_sum<1>(0, f.nprev, f.prev, tot);
+  const double alpha = rho / tot[0];  // cg.cpp:107-108
+  if (blockIdx.x == 0 && threadIdx.x == 0 && !st->done) {
+    st->pq = tot[0];
+    st->alpha = alpha;
+  }
+  return alpha;
+}
+
+// ---------------------------------------------------------------------------
 // y = A x   (Scalar::operator=(A_x), scalar_operators.cpp:49-72)
 // ---------------------------------------------------------------------------
 template <typename T, int V, bool SYM>
@@ -77,7 +482,7 @@ __global__ __launch_bounds__(kBlock) void k_resid(Grid g, DMat<T> A, const T *b,
 
 // ---------------------------------------------------------------------------
 // Krylov start: r = b - A x with its norms, and per MODE
-//   0 diagonal CG: rho = r.(r/c)        (cg.cpp:47-80)
+//   0 diagonal CG: rho = r.(r/c)        (cg.cpp:47-80), z = r/c into aux if given
 //   1 preconditioned CG: e1 = omega r / c into aux
 //   2 BiCGS: r~ = r into aux, rho = r~.r (bicgs.cpp:53-84)
 // partials: sum r^2/dV^2, sum r^2, rho
@@ -100,13 +505,14 @@ __global__ __launch_bounds__(kBlock) void k_start(Grid g, DMat<T> A, Metric m, c
     if (MODE == 0) {
       T z = R.v[q] * (T(1) / G.c.v[q]);
       acc[2] += (double)(R.v[q] * z);
+      E.v[q] = z;
     } else if (MODE == 1) {
       E.v[q] = omega * R.v[q] / G.c.v[q];
     } else {
       acc[2] += rd * rd;
     }
   }
-  if (MODE == 1) stv<T, V>(aux + P, E);
+  if (MODE == 1 || (MODE == 0 && aux)) stv<T, V>(aux + P, E);
   if (MODE == 2) stv<T, V>(aux + P, R);
   PSB_TILE_END
   block_partial<3>(acc, w.partial);
@@ -176,11 +582,12 @@ __global__ __launch_bounds__(kBlock) void k_cg_pq(Grid g, DMat<T> A, const T *r_
   stv<T, V>(r + P, R);                                        \
   if (!DIAG) stv<T, V>(e1 + P, E);
 
-template <typename T, int V, bool DIAG>
+// (get_alpha gives alpha, or false where the solve has stopped; in FP64 it is
+// called once the first loads are under way)
+template <typename T, int V, bool DIAG, class GetAlpha>
 __device__ __forceinline__ void cg_xr_body(Span sp, const Grid &g, const T *c, const Metric &m,
                                            const T *p, const T *q, T *x, T *r, T *e1, T omega,
-                                           const DevState *st, Work w) {
-  const T alpha = (T)st->alpha;
+                                           const DevState *st, Work w, GetAlpha get_alpha) {
   // the reference norm's sum (dV loads, two FP64 divisions per cell) only
   // when the solve stops on it
   const bool vd = st->norm == 0;
@@ -196,6 +603,9 @@ __device__ __forceinline__ void cg_xr_body(Span sp, const Grid &g, const T *c, c
     const int Pf = (qq < q1 ? qq : 0) * V;
     VecN<T, V> Xn = ldv<T, V>(x + Pf), Rn = ldv<T, V>(r + Pf), Pn = ldv<T, V>(p + Pf),
                Qn = ldv<T, V>(q + Pf), Cn = ldv<T, V>(c + Pf);
+    double al;
+    if (!get_alpha(al)) return;
+    const T alpha = (T)al;
     for (; qq < q1; qq += kBlock) {
       const int P = qq * V;
       int i, j, k;
@@ -210,6 +620,9 @@ __device__ __forceinline__ void cg_xr_body(Span sp, const Grid &g, const T *c, c
       PSB_CG_XR_CELL
     }
   } else {
+    double al;
+    if (!get_alpha(al)) return;
+    const T alpha = (T)al;
     PSB_SPAN_BEGIN(g, V, sp)
     VecN<T, V> X = ldv<T, V>(x + P), R = ldv<T, V>(r + P), Pp = ldv<T, V>(p + P),
                Q = ldv<T, V>(q + P), C = ldv<T, V>(c + P), E;
@@ -223,9 +636,170 @@ __device__ __forceinline__ void cg_xr_body(Span sp, const Grid &g, const T *c, c
 template <typename T, int V, bool DIAG>
 __global__ __launch_bounds__(kBlock) void k_cg_xr(Grid g, const T *c, Metric m, const T *p,
                                                   const T *q, T *x, T *r, T *e1, T omega,
-                                                  DevState *st, Work w) {
-  if (st->done) return;
-  cg_xr_body<T, V, DIAG>(grid_span(), g, c, m, p, q, x, r, e1, omega, st, w);
+                                                  DevState *st, Work w, Fold f) {
+  cg_xr_body<T, V, DIAG>(grid_span(), g, c, m, p, q, x, r, e1, omega, st, w, [&](double &al) {
+    const int done = st->done;
+    const double rho = st->rho;
+    al = f.nprev > 0 ? fold_pq(f, st, rho) : st->alpha;
+    return done == 0;
+  });
+}
+
+// ---------------------------------------------------------------------------
+// CG step 1 with the diagonal preconditioner on small grids, FP64: the step
+// FIN_XR_DIAG of the iteration before folded in (f.nprev > 0), and everything
+// a cell vector needs -- z and p at its seven points, the couplings --
+// loaded before it, so that the two round trips to memory are one.  z = r / c
+// comes from k_cg_xr_di (k_start in the first iteration): forming it here, at
+// seven points with a division each, took 7.4 against 5.9 us at 64^3.  What
+// bounds it is that latency: at 64^3 a thread has one vector.  Same partition
+// into blocks as the kernels it stands in for (ntiles > 0: k_cg_pq_march's
+// tiles and slabs of TI planes; else k_cg_pq's spans), same gather: the
+// results are theirs bit for bit.
+// ---------------------------------------------------------------------------
+template <int V>
+struct PreX {  // the operand at the seven points
+  VecN<double, V> own, w, e, s, n;
+  double b, t;
+  int j, k;
+  __device__ __forceinline__ VecN<double, V> vec(int, int, int, int) const { return own; }
+  __device__ __forceinline__ double at(int, int, int, int kk) const { return kk > k ? t : b; }
+};
+template <int V>
+__device__ __forceinline__ VecN<double, V> x_nbj(const PreX<V> &x, int, int, int jj, int) {
+  return jj > x.j ? x.n : x.s;
+}
+template <int V>
+__device__ __forceinline__ VecN<double, V> x_nbi(const PreX<V> &x, bool up, int, int, int, int) {
+  return up ? x.e : x.w;
+}
+
+// an array at the seven points (a point outside the domain: the cell itself)
+template <int V>
+struct Seven {
+  VecN<double, V> v[5];
+  double b, t;
+  __device__ __forceinline__ void load(const double *a, const Grid &g, int P, int i, int j, int k) {
+    v[0] = ldv<double, V>(a + P);
+    v[1] = ldv<double, V>(a + (i > 0 ? P - g.sI : P));
+    v[2] = ldv<double, V>(a + (i < g.nx - 1 ? P + g.sI : P));
+    v[3] = ldv<double, V>(a + (j > 0 ? P - g.nz : P));
+    v[4] = ldv<double, V>(a + (j < g.ny - 1 ? P + g.nz : P));
+    b = a[k > 0 ? P - 1 : P];
+    t = a[k + V < g.nz ? P + V : P];
+  }
+};
+
+// CG step 2 with the diagonal preconditioner on the same grids: FIN_PQ folded
+// in, the vector's five arrays and its cell sizes loaded before it; z = r / c,
+// which the rho partials need anyway, left in q for the next p/q step
+template <int V>
+__global__ __launch_bounds__(kBlock) PSB_SMALL void k_cg_xr_di(Grid g, const double *c, Metric m,
+                                                               const double *p, double *q,
+                                                               double *x, double *r, DevState *st,
+                                                               Work w, Fold f) {
+  const int nvec = g.N / V;
+  const Span sp = grid_span();
+  const int per = (nvec + sp.nb - 1) / sp.nb;
+  const int q0 = sp.bl * per + (int)threadIdx.x, q1 = min(sp.bl * per + per, nvec);
+  const int done = st->done, norm = st->norm;
+  const double rho = st->rho;
+  VecN<double, V> X, R, Pp, Q, C;
+  double dv[V];
+  auto load = [&](int qq) {
+    const int P = qq * V;
+    int i, j, k;
+    g.ijk(P, i, j, k);
+    X = ldv<double, V>(x + P);
+    R = ldv<double, V>(r + P);
+    Pp = ldv<double, V>(p + P);
+    Q = ldv<double, V>(q + P);
+    C = ldv<double, V>(c + P);
+#pragma unroll
+    for (int u = 0; u < V; u++) dv[u] = m.dV(i, j, k + u);
+  };
+  load(q0 < q1 ? q0 : 0);
+  const double alpha = f.nprev > 0 ? fold_pq(f, st, rho) : st->alpha;
+  if (done) return;
+  double acc[3] = {0.0, 0.0, 0.0};
+  for (int qq = q0; qq < q1; qq += kBlock) {
+    if (qq != q0) load(qq);
+#pragma unroll
+    for (int u = 0; u < V; u++) {
+      X.v[u] = X.v[u] + alpha * Pp.v[u];
+      R.v[u] = R.v[u] - alpha * Q.v[u];
+      const double rd = R.v[u];
+      if (norm == 0) acc[0] += rd * rd / dv[u] / dv[u];
+      acc[1] += rd * rd;
+      const double z = R.v[u] * (1.0 / C.v[u]);
+      acc[2] += R.v[u] * z;
+      Q.v[u] = z;
+    }
+    stv<double, V>(x + qq * V, X);
+    stv<double, V>(r + qq * V, R);
+    stv<double, V>(q + qq * V, Q);
+  }
+  block_partial<3>(acc, w.partial);
+}
+
+template <int V, bool SYM>
+__global__ __launch_bounds__(kBlock) PSB_SMALL void k_cg_pq_di(Grid g, DMat<double> A,
+                                                               const double *z,
+                                                               const double *pold, double *pnew,
+                                                               double *q, const DevState *st,
+                                                               Fold f, Work w, int TI,
+                                                               int ntiles) {
+  const StopIn si(st);
+  double beta = st->beta;
+  const int nvec = g.N / V, nv = g.nz / V;
+  // this thread's vectors: q0, q0 + step, ... below q1
+  int q0, q1, step;
+  const Span sp = grid_span();
+  if (ntiles > 0) {
+    const int slab = sp.bl / ntiles, t = (sp.bl - slab * ntiles) * kBlock + (int)threadIdx.x;
+    const int i0 = slab * TI, i1 = min(i0 + TI, g.nx);
+    step = g.ny * nv;
+    q0 = i0 * step + t;
+    q1 = t < step ? i1 * step : q0;
+  } else {
+    const int per = (nvec + sp.nb - 1) / sp.nb;
+    step = kBlock;
+    q0 = sp.bl * per + (int)threadIdx.x;
+    q1 = min(sp.bl * per + per, nvec);
+  }
+  Seven<V> Z, Q;
+  Coef<double, V, SYM> cf;
+  int P, i, j, k;
+  auto load = [&](int qq) {
+    P = qq * V;
+    g.ijk(P, i, j, k);
+    Z.load(z, g, P, i, j, k);
+    Q.load(pold, g, P, i, j, k);
+    cf = load_coef<double, V, SYM>(g, A, P, i, j, k);
+  };
+  load(q0 < q1 ? q0 : 0);
+  if (f.nprev > 0 ? fold_xr_diag(f, si, st, beta) : si.done != 0) return;
+  double acc[1] = {0.0};
+  for (int qq = q0; qq < q1; qq += step) {
+    if (qq != q0) load(qq);
+    PreX<V> px;
+    px.j = j;
+    px.k = k;
+    VecN<double, V> *const o[5] = {&px.own, &px.w, &px.e, &px.s, &px.n};
+#pragma unroll
+    for (int h = 0; h < 5; h++)
+#pragma unroll
+      for (int u = 0; u < V; u++) o[h]->v[u] = Z.v[h].v[u] + beta * Q.v[h].v[u];
+    px.b = Z.b + beta * Q.b;
+    px.t = Z.t + beta * Q.t;
+    const Gath<double, V> G = gather_c<double, V, SYM>(g, cf, px, P, i, j, k);
+    const VecN<double, V> Y = apply_A<double, V>(G);
+    stv<double, V>(pnew + P, G.x);
+    stv<double, V>(q + P, Y);
+#pragma unroll
+    for (int u = 0; u < V; u++) acc[0] += (double)(G.x.v[u] * Y.v[u]);
+  }
+  block_partial<1>(acc, w.partial);
 }
 
 // ---------------------------------------------------------------------------
@@ -891,291 +1465,6 @@ __global__ __launch_bounds__(kBlock) void k_abi_x(Grid g, Metric m, const T *z1,
   }
   PSB_TILE_END
   block_partial<3>(acc, w.partial);
-}
-
-// ---------------------------------------------------------------------------
-// pass 2 of the reductions: one block sums the partials of the kernel
-// before it (fixed order) and applies the scalar step
-// ---------------------------------------------------------------------------
-enum FinOp {
-  FIN_START_DIAG, FIN_START_AC, FIN_START_BICGS, FIN_PQ, FIN_XR_DIAG, FIN_XR_AC, FIN_RHO,
-  FIN_XR_RU, FIN_IR_RESID, FIN_CENTER, FIN_RELRES, FIN_BI1, FIN_BI2, FIN_BI3, FIN_RU_START,
-  FIN_RU, FIN_RU_END, FIN_ACMEAN, FIN_ACRES, FIN_RHO_FLEX
-};
-
-// stop logic shared by the Krylov loops (cg.cpp:121-160, bicgs.cpp:174-210),
-// after iteration st->iter with the new residual
-__device__ inline void krylov_stop(DevState *st, double res, bool small_omega) {
-  const int i = st->iter;
-  st->res = res;
-  if (st->hist && i + 1 < st->hist_cap) st->hist[i + 1] = res;
-  int done = 0, conv = 0, reason = 0;
-  if (!(res == res) || res > 1e300) {
-    done = 1; reason = 8;
-  } else if (res < st->res_tol && i >= st->mini - 1) {
-    done = 1; conv = 1; reason = 1;
-  } else if (res < st->res0 * st->res_rat && i >= st->mini - 1) {
-    done = 1; conv = 1; reason = 2;
-  } else if (small_omega) {
-    done = 1; reason = 6;
-  } else if (st->stalecount > 0) {
-    bool stale = true;
-    for (int q = 0; q < st->stalecount; q++)
-      if (res < st->stale[q]) { stale = false; break; }
-    if (stale) {
-      done = 1; reason = 3;
-    } else {
-      for (int q = 0; q + 1 < st->stalecount; q++) st->stale[q] = st->stale[q + 1];
-      st->stale[st->stalecount - 1] = res;
-    }
-  }
-  if (done) {
-    st->report_iters = i + 1;
-  } else if (i + 1 >= st->maxit) {
-    done = 1;
-    st->report_iters = st->maxit + 1;
-  }
-  st->converged = conv;
-  st->reason = reason;
-  st->iter = i + 1;
-  st->done = done;
-}
-
-__device__ inline double ref_norm(const DevState *st, double sum_voldiv) {
-  // sqrt(dot_voldiv_avg)/scale with dot_voldiv_avg = d/ntot/ntot
-  // (scalar.h:317-326, cg.cpp:121)
-  double d = sum_voldiv / st->ntot;
-  d = d / st->ntot;
-  return sqrt(d) / st->scale;
-}
-
-__device__ inline void krylov_init(DevState *st, double res, double rsq, double rho) {
-  st->res0 = res;
-  st->res = res;
-  st->rsq0 = rsq;
-  st->rsq = rsq;
-  st->rho = rho;
-  st->beta = 0.0;
-  st->zmean = 0.0;
-  st->iter = 0;
-  st->report_iters = 0;
-  st->converged = 0;
-  st->reason = 0;
-  st->done = 0;
-  if (st->hist && st->hist_cap > 0) st->hist[0] = res;
-  for (int q = 0; q < st->stalecount && q < kStaleMax; q++) st->stale[q] = 1.0e24;
-  if (st->stalecount > 0) st->stale[st->stalecount - 1] = res;
-}
-
-// steps of a finished loop (or a refresh not pending) do nothing
-__device__ inline bool fin_skip(int op, const DevState *st) {
-  switch (op) {
-    case FIN_PQ: case FIN_XR_DIAG: case FIN_XR_AC: case FIN_RHO: case FIN_RHO_FLEX:
-    case FIN_XR_RU:
-    case FIN_BI1: case FIN_BI2: case FIN_BI3:
-      return st->done != 0;
-    case FIN_RU:
-      return st->done || !st->update;
-    default:
-      return false;
-  }
-}
-
-// sum of the partials of blocks [b0, b0 + nblk) in a fixed order (all
-// threads of the block receive the totals)
-template <int NR>
-__device__ inline void fin_sum(int b0, int nblk, const double *partial, double (&acc)[NR]) {
-  __shared__ double sm[kWaves][NR];
-#pragma unroll
-  for (int r = 0; r < NR; r++) acc[r] = 0.0;
-  for (int q = threadIdx.x; q < nblk; q += kBlock) {
-#pragma unroll
-    for (int r = 0; r < NR; r++) acc[r] += partial[(size_t)(b0 + q) * NR + r];
-  }
-  block_sum<NR>(acc, sm);
-}
-
-// the scalar step of op on the totals (one thread)
-__device__ inline void fin_apply(int op, const double *tot, DevState *st, DevState *st2,
-                                 double *out) {
-  switch (op) {
-    case FIN_START_DIAG:
-    case FIN_START_AC:
-    case FIN_START_BICGS: {
-      const double res = st->norm == 0 ? ref_norm(st, tot[0]) : sqrt(tot[1]);
-      krylov_init(st, res, tot[1], tot[2]);
-      if (res < st->res_tol) {  // cg.cpp:64, bicgs.cpp:70 early return
-        st->done = 1;
-        st->converged = 1;
-        st->reason = 7;
-      }
-      if (!(res == res)) {
-        st->done = 1;
-        st->reason = 8;
-      }
-      if (op == FIN_START_BICGS && !st->done && sqrt(fabs(tot[2])) < st->res_tol) {
-        st->done = 1;  // bicgs.cpp:89 at i = 0
-        st->reason = 4;
-        st->report_iters = 1;
-      }
-      break;
-    }
-    case FIN_PQ:
-      st->pq = tot[0];
-      st->alpha = st->rho / tot[0];  // cg.cpp:107-108
-      break;
-    case FIN_XR_DIAG:
-    case FIN_XR_AC: {
-      const double res = st->norm == 0 ? ref_norm(st, tot[0]) : sqrt(tot[1]);
-      st->rsq = tot[1];
-      krylov_stop(st, res, false);
-      if (op == FIN_XR_DIAG && !st->done) {
-        st->beta = tot[2] / st->rho;  // cg.cpp:93
-        st->rho = tot[2];
-      }
-      break;
-    }
-    case FIN_XR_RU: {  // FP32 step inside the refinement: refresh or stop
-      const double res = sqrt(tot[1]);
-      const int i = st->iter;
-      st->rsq = tot[1];
-      st->res = res;
-      st->iter = i + 1;
-      if (!(res == res) || res > 1e300) {
-        st->done = 1;
-        st->reason = 8;
-        st->report_iters = i + 1;
-      } else if (res < st->rlast * st->delta || res < sqrt(st->rsq0) * st->res_rat) {
-        st->update = 1;
-      } else if (i + 1 >= st->maxit) {
-        st->done = 1;
-        st->report_iters = st->maxit + 1;
-      }
-      break;
-    }
-    case FIN_RU_START:
-    case FIN_RU: {  // true residual after a refresh (or at the start)
-      const double rl2 = sqrt(tot[0]);
-      const double res = st->norm == 0 ? ref_norm(st, tot[1]) : rl2;
-      if (op == FIN_RU_START) {
-        krylov_init(st, res, tot[0], 0.0);
-        st->outer = 0;
-      } else {
-        st->outer += 1;
-        if (st->hist && st->outer < st->hist_cap) st->hist[st->outer] = res;
-      }
-      st->res_true = res;
-      st->rl2_true = rl2;
-      if (op == FIN_RU_START) st->bsq = tot[3];
-      st->rlast = rl2;
-      st->update = 0;
-      st->res = sqrt(tot[2]);
-      if (!(res == res)) {
-        st->done = 1;
-        st->reason = 8;
-      } else if (res < st->res_tol || res < st->res0 * st->res_rat || st->res0 == 0.0) {
-        st->done = 1;
-        st->converged = 1;
-        st->reason = 2;
-        st->report_iters = st->iter;
-      } else if (st->iter >= st->maxit) {
-        st->done = 1;
-        st->report_iters = st->maxit + 1;
-      }
-      break;
-    }
-    case FIN_ACMEAN:  // mean of the restricted right-hand side over active cells
-      st->mean[0] = tot[1] > 0.0 ? tot[0] / tot[1] : 0.0;
-      break;
-    case FIN_ACRES: {  // AC::residual: sqrt(dot_voldiv_avg(r, r)) * dt (scale = dt)
-      double d = tot[0] / st->ntot;
-      d = d / st->ntot;
-      out[0] = sqrt(d) * st->scale;
-      break;
-    }
-    case FIN_RU_END:  // true residual at exit without convergence
-      st->res_true = st->norm == 0 ? ref_norm(st, tot[1]) : sqrt(tot[0]);
-      st->rl2_true = sqrt(tot[0]);
-      break;
-    case FIN_RHO:
-    case FIN_RHO_FLEX: {
-      const double m = !st->keepmean && tot[3] > 0.0 ? tot[1] / tot[3] : 0.0;
-      const double rho = tot[0] - m * tot[2];
-      st->zmean = m;
-      if (st->iter == 0) {
-        st->beta = 0.0;
-      } else if (op == FIN_RHO) {
-        st->beta = rho / st->rho;  // Fletcher-Reeves, cg.cpp:93
-      } else {
-        // flexible: beta = -z'.A p / p.A p with z' = z - m on the active
-        // cells, so the new direction is A-orthogonal to the last one
-        // whatever the preconditioner did (Notay, SISC 22 (2000) 1444-1460)
-        const double zq = tot[4] - m * tot[5];
-        st->beta = st->pq != 0.0 ? -zq / st->pq : 0.0;
-      }
-      st->rho = rho;
-      break;
-    }
-    case FIN_IR_RESID:  // st: FP64 outer state, st2: FP32 inner state
-      st->rsq = tot[0];
-      st->res = st->norm == 0 ? ref_norm(st, tot[1]) : sqrt(tot[0]);
-      st2->mean[0] = !st2->keepmean && tot[3] > 0.0 ? tot[2] / tot[3] : 0.0;
-      break;
-    case FIN_CENTER: {
-      krylov_init(st, sqrt(tot[0]), tot[0], 0.0);
-      if (tot[0] == 0.0) st->done = 1;
-      break;
-    }
-    case FIN_RELRES:
-      out[0] = tot[0];
-      out[1] = tot[1];
-      break;
-    case FIN_BI1:
-      st->rv = tot[0];
-      st->alpha = st->rho / tot[0];  // bicgs.cpp:122-123
-      break;
-    case FIN_BI2:
-      st->rv_ss = tot[0];
-      st->rv_ts = tot[1];
-      st->rv_tt = tot[2];
-      st->omega = tot[1] / tot[2];  // bicgs.cpp:155-157
-      break;
-    case FIN_BI3: {
-      if (sqrt(st->rv_ss) < st->res_tol) {  // bicgs.cpp:134-138
-        st->done = 1;
-        st->converged = 0;
-        st->reason = 5;
-        st->report_iters = st->iter + 1;
-        break;
-      }
-      const double res = st->norm == 0 ? ref_norm(st, tot[0]) : sqrt(tot[1]);
-      st->rsq = tot[1];
-      const bool small_om = st->omega >= -st->res_tol && st->omega <= st->res_tol;
-      krylov_stop(st, res, small_om);
-      if (!st->done) {
-        // top of the next iteration: rho = r~.r, breakdown test (bicgs.cpp:84-89)
-        const double rho = tot[2];
-        if (sqrt(fabs(rho)) < st->res_tol) {
-          st->done = 1;
-          st->reason = 4;
-          st->report_iters = st->iter + 1;
-        } else {
-          st->beta = (rho / st->rho) * (st->alpha / st->omega);  // bicgs.cpp:102
-          st->rho = rho;
-        }
-      }
-      break;
-    }
-  }
-}
-
-template <int NR>
-__global__ __launch_bounds__(kBlock) void k_finalize(int op, int nblk, const double *partial,
-                                                     DevState *st, DevState *st2, double *out) {
-  if (fin_skip(op, st)) return;
-  double acc[NR];
-  fin_sum<NR>(0, nblk, partial, acc);
-  if (threadIdx.x == 0) fin_apply(op, acc, st, st2, out);
 }
 
 // ---------------------------------------------------------------------------
