@@ -584,8 +584,8 @@ def main():
                       "matrix copy, marching)",
              "sweep_last": "k_jacobi_march<float,4,-,RHO,_Float16,flux> (last post-sweep with "
                            "the rho partials, marching)",
-             "restrict": "k_restrict_march<float,4,...> (residual block sums, coarse first "
-                         "sweep fused)",
+             "restrict": "k_pre_restrict<float,4,_Float16,flux> (last pre-sweep, residual block "
+                         "sums and the coarse level's first sweep in one pass)",
              "cg_xr": "k_cg_xr<float,4> (x, r update, norms, next first sweep)"}
     # isolated back-to-back launches of the fine-level sweep and SpMVs
     ms_j, by_j = s.time_kernel(2, reps=50)

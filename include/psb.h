@@ -512,7 +512,8 @@ enum psb_kernel_kind {
   PSB_K_SWEEP = 0,    /* damped Jacobi sweep (pre-smoothing, later post-sweeps) */
   PSB_K_SWEEP_PROL,   /* first post-sweep, prolongation of the coarse correction fused */
   PSB_K_SWEEP_LAST,   /* last post-sweep of the finest level, the rho partials fused */
-  PSB_K_RESTRICT,     /* residual block sums to level 1, its first sweep fused */
+  PSB_K_RESTRICT,     /* residual block sums to level 1, its first sweep fused (with the
+                         last pre-sweep where both are one pass)              */
   PSB_K_CG_PQ,        /* p = z + beta p, q = A p, p.q */
   PSB_K_CG_XR,        /* x += alpha p, r -= alpha q, norms, next first sweep */
   PSB_K_RU_RESID,     /* FP64 true residual of a reliable update (gated) */

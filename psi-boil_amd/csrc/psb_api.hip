@@ -30,6 +30,7 @@
 #include "psb_march.h"
 #include "psb_lds.h"
 #include "psb_tail.h"
+#include "psb_two.h"
 #include "psb_internal.h"
 
 // FP32 levels evaluate the stencil in flux form (set to 0 for the plain form)
@@ -511,6 +512,87 @@ void restrict_(psb_ctx *C, const Level<T> &f, const T *e, Level<T> &cL, T omega,
     else if (cL.CJ == 2) restrict_k<T, V, 1, 2>(C, f, e, cL, omega, st);
     else restrict_k<T, V, 1, 1>(C, f, e, cL, omega, st);
   });
+}
+
+// ---------------------------------------------------------------------------
+// two stages of a level in one pass (psb_two.h)
+// ---------------------------------------------------------------------------
+// Tile and slab for a level: rows whole where four of them fit a block, else
+// split along k; of the row counts and slab depths the cheapest by
+//   rounds of blocks over the CUs * planes per block * waves on a CU
+// (what the redundant rows and planes cost against CUs without a block;
+// measured at 256^3, FP32: R = 8 and 32 planes, one block per CU, 90 us, R = 8
+// and 16 planes 97, R = 4 and 64 planes 106, R = 10 and 28 planes, 260 blocks,
+// 127).  The registers allow 3 waves per SIMD.
+template <typename T>
+bool two_shape(const psb_ctx *C, const Grid &g, TwoShape &s) {
+  constexpr int V = vmax<T>();
+  if (!C->two || g.nz % V != 0) return false;
+  const int nv = g.nz / V;
+  double best = 0.0;
+  for (const int KO : {nv, 64, 32, 16}) {
+    if (KO > nv || (KO != nv && best > 0.0)) continue;
+    const int KT = KO == nv ? nv : KO + 2, ntk = (nv + KO - 1) / KO;
+    for (int R = 2; (R + 2) * KT <= kTwoThreads; R += 2) {
+      const size_t lds = (size_t)(2 * (R + 4) + 2 * (R + 2) + R) * KT * V;
+      if (lds * sizeof(T) > 150 * 1024) break;
+      const int waves = ((R + 2) * KT + 63) / 64, per_cu = std::max(1, 12 / waves);
+      const long long nt = (long long)((g.ny + R - 1) / R) * ntk;
+      for (int TI = 2; TI < g.nx + 2; TI += 2) {
+        const long long nb = nt * ((g.nx + TI - 1) / TI);
+        const long long rounds = (nb + 256 * per_cu - 1) / (256 * per_cu);
+        const long long act = std::min<long long>(per_cu, (nb + 255) / 256);
+        const double cost = (double)rounds * (TI + 2) * (4 + waves * act);
+        if (nb >= (1 << 30) || (best > 0.0 && cost >= best)) continue;
+        best = cost;
+        s.RT = R + 2;
+        s.KT = KT;
+        s.KO = KO;
+        s.ntj = (g.ny + R - 1) / R;
+        s.ntk = ntk;
+        s.lds = lds;
+        s.TI = TI;
+        s.nblocks = (int)nb;
+        s.threads = waves * 64;
+      }
+    }
+  }
+  return best > 0.0;
+}
+
+// the last pre-sweep of level lv (e to eout) and the restriction to cL in one
+// pass; false where the level does not suit it
+template <typename T, typename M, bool FLUX>
+void pre_restrict_m(psb_ctx *C, const Level<T> &lv, DMat<M> A, const T *e, T *eout, Level<T> &cL,
+                    T omega, T omegaH, DevState *st, const TwoShape &s) {
+  constexpr int V = vmax<T>();
+  auto go = [&](auto ck) {
+    hipLaunchKernelGGL((k_pre_restrict<T, V, M, FLUX, decltype(ck)::value>), dim3(s.nblocks),
+                       dim3(s.threads), s.lds * sizeof(T), C->stream, lv.g, A, lv.r, e, eout,
+                       lv.aflag, cL.g, cL.c, cL.aflag, cL.r, cL.e[0], omega, omegaH, st, s);
+  };
+  if (cL.CK == 2) go(std::integral_constant<int, 2>());
+  else go(std::integral_constant<int, 1>());
+}
+template <typename T>
+bool pre_restrict(psb_ctx *C, const Level<T> &lv, const T *e, T *eout, Level<T> &cL, T omega,
+                  T omegaH, DevState *st) {
+  TwoShape s{};
+  if (lv.ae || cL.CI != 2 || cL.CJ != 2 || !two_shape<T>(C, lv.g, s)) return false;
+  if (std::is_same<T, float>::value && !lv.d) return false;
+  // four coefficient arrays, r, e in, e out; the coarse cells' c, r and e
+  ProbeScope ps(C, PSB_K_RESTRICT, lv.g,
+                4.0 * (lv.h16() ? 2 : sizeof(T)) + 3.0 * sizeof(T) + (lv.aflag ? 1 : 0) +
+                    (3.0 * sizeof(T) + (cL.aflag ? 1 : 0)) / (4 * cL.CK));
+  if constexpr (std::is_same<T, float>::value) {
+    if (lv.h16())
+      pre_restrict_m<T, _Float16, true>(C, lv, lv.mat16(), e, eout, cL, omega, omegaH, st, s);
+    else
+      pre_restrict_m<T, T, true>(C, lv, lv.matflux(), e, eout, cL, omega, omegaH, st, s);
+  } else {
+    pre_restrict_m<T, T, false>(C, lv, lv.mat(), e, eout, cL, omega, omegaH, st, s);
+  }
+  return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -1208,15 +1290,20 @@ T *vcycle(psb_ctx *C, Hier<T> &H, int l, DevState *st, int nu1, int nu2, T omega
   if (!kcycle_level(C, H, l) && tail_at(C, H, l))
     return tail_cycle<T>(C, H, l, nu1, nu2, omega, cfac, false);
   int cur = done;
-  for (int s = 1 + done; s < nu1; s++) {
-    jacobi<T, false>(C, lv, lv.e[cur], lv.e[(cur + 1) % 3], nullptr, nullptr, T(0), omega, st);
-    cur = (cur + 1) % 3;
-  }
   Level<T> &cL = H.L[l + 1];
+  bool restricted = false;
+  for (int s = 1 + done; s < nu1; s++) {
+    const int nxt = (cur + 1) % 3;
+    if (s == nu1 - 1)
+      restricted = pre_restrict<T>(C, lv, lv.e[cur], lv.e[nxt], cL, omega, T(omega / cL.scale), st);
+    if (!restricted)
+      jacobi<T, false>(C, lv, lv.e[cur], lv.e[nxt], nullptr, nullptr, T(0), omega, st);
+    cur = nxt;
+  }
   // corrections on a level with a scaled half-precision matrix are held
   // divided by its scale: the coarse level's first sweep, the prolongation
   // and the preconditioner's output carry the ratios
-  restrict_<T>(C, lv, lv.e[cur], cL, T(omega / cL.scale), st);
+  if (!restricted) restrict_<T>(C, lv, lv.e[cur], cL, T(omega / cL.scale), st);
   const bool kc = kcycle_level(C, H, l + 1);  // the Krylov steps choose the scaling
   T *zH = kc ? kstep<T>(C, H, l + 1, st, nu1, nu2, omega, cfac)
              : vcycle<T>(C, H, l + 1, st, nu1, nu2, omega, cfac);
@@ -2706,6 +2793,7 @@ int psb_create(psb_ctx **out, const psb_layout *L) {
     if (std::getenv("PSB_NO_KFUSE")) C->kfuse = false;
     if (std::getenv("PSB_NO_TAIL")) C->tail = false;
     if (std::getenv("PSB_NO_FOLD")) C->fold = false;
+    if (std::getenv("PSB_NO_TWO")) C->two = false;
     if (std::getenv("PSB_NO_LDS")) {
       C->lds32 = C->lds64 = 0;
     } else if (const char *m = std::getenv("PSB_LDS_MASK")) {

@@ -287,6 +287,9 @@ struct psb_ctx {
   // CG-di's stop test and beta in the p/q step on small grids (PSB_NO_FOLD
   // set: a launch of their own, for comparisons)
   bool fold = true;
+  // two stages of a level in one pass (psb_two.h; PSB_NO_TWO set: one kernel
+  // each, for comparisons)
+  bool two = true;
   // the pressure's boundary conditions for the device assembly (all Neumann,
   // value 0: walls) and the boundary source it formed (NULL: none)
   psb_bnd bnd{};
