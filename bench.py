@@ -582,8 +582,8 @@ def main():
                            "the prolongation fused; FP16 matrix copy, LDS-staged)",
              "sweep": "k_jacobi_march<float,4,-,-,_Float16,flux> (damped Jacobi sweep, FP16 "
                       "matrix copy, marching)",
-             "sweep_last": "k_jacobi_march<float,4,-,RHO,_Float16,flux> (last post-sweep with "
-                           "the rho partials, marching)",
+             "sweep_last": "k_post_two<float,4,_Float16,flux,RHO> (both post-sweeps with the "
+                           "prolongation and the rho partials in one pass)",
              "restrict": "k_pre_restrict<float,4,_Float16,flux> (last pre-sweep, residual block "
                          "sums and the coarse level's first sweep in one pass)",
              "cg_xr": "k_cg_xr<float,4> (x, r update, norms, next first sweep)"}

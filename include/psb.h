@@ -133,10 +133,9 @@ typedef struct {
                             operator on level 0 (its q = A p reads 8 instead
                             of 16 B per cell; the FP64 reliable updates
                             still measure the true residual)                */
-  int ac_fuse;           /* PSB_MIXED: 1 runs the two post-sweeps of a level
-                            in one pass (2.5-D marching tile) where the
-                            level's shape allows; 0 one kernel per sweep
-                            (default: faster on MI355X today; same z)      */
+  int ac_fuse;           /* accepted and without effect: the two post-sweeps
+                            of a level run in one pass wherever its shape
+                            allows                                         */
   int ac_kcycle;         /* K-cycle levels, bit l for level l (level 1 is the
                             first coarse level; bit 0 must be 0): there the
                             coarse correction is two flexible-CG steps
@@ -486,8 +485,8 @@ int psb_batch_solve_device(psb_batch *bt, double *const *d_x,
  * 0 FP64 SpMV, 1 FP32 SpMV, 2 FP32 damped Jacobi sweep on the fine level as
  * the last mixed-precision solve set it up (flux form; FP16 matrix copy with
  * ac_store = 1), 3 plain FP32 copy of the grid (reference stream for
- * hardware byte counters), 4 the fine level's two post-sweeps in one pass
- * (ac_fuse = 1 form), 5 the same two sweeps as two kernels, 6 the FP32 CG
+ * hardware byte counters), 4 the fine level's two post-sweeps in one pass,
+ * 5 the same two sweeps as two kernels, 6 the FP32 CG
  * p/q step of the mixed multigrid-preconditioned solve on the fine level,
  * 7 the fine level's first post-sweep with the prolongation fused in, 8 its
  * last post-sweep with the rho partials of the flexible beta, 9 the FP32 CG
@@ -511,7 +510,8 @@ int psb_time_kernel(psb_ctx *ctx, int kernel, int reps, double *avg_ms,
 enum psb_kernel_kind {
   PSB_K_SWEEP = 0,    /* damped Jacobi sweep (pre-smoothing, later post-sweeps) */
   PSB_K_SWEEP_PROL,   /* first post-sweep, prolongation of the coarse correction fused */
-  PSB_K_SWEEP_LAST,   /* last post-sweep of the finest level, the rho partials fused */
+  PSB_K_SWEEP_LAST,   /* last post-sweep of the finest level, the rho partials fused (with
+                         the first where both are one pass)                   */
   PSB_K_RESTRICT,     /* residual block sums to level 1, its first sweep fused (with the
                          last pre-sweep where both are one pass)              */
   PSB_K_CG_PQ,        /* p = z + beta p, q = A p, p.q */

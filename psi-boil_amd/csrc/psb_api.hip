@@ -26,7 +26,6 @@
 #include <vector>
 
 
-#include "psb_fused.h"
 #include "psb_march.h"
 #include "psb_lds.h"
 #include "psb_tail.h"
@@ -390,53 +389,6 @@ void jacobi(psb_ctx *C, const Level<T> &lv, const T *e, T *eout, const Level<T> 
   jacobi_m<T, RHO, T, false>(C, lv, lv.mat(), e, eout, coarse, eH, cfac, omega, zscale, st, qf);
 }
 
-// the two post-sweeps of level lv in one pass (k_post2): the first with the
-// prolongation of eH from `coarse`, the second writing eout (and the rho
-// partials when RHO).  False when the level's shape does not suit it.
-template <bool RHO, typename M, bool FLUX>
-void post2_m(psb_ctx *C, const Level<float> &lv, DMat<M> A, const float *e, float *eout,
-             const Level<float> &coarse, const float *eH, float cfac, float omega, float zscale,
-             DevState *st, const FuseShape &f, const float *qf) {
-  ProlX<float, 4> pr{};
-  pr.e = e;
-  pr.eH = eH;
-  pr.af = lv.aflag;
-  pr.cfac = cfac;
-  pr.sI = coarse.CI == 2 ? 1 : 0;
-  pr.sJ = coarse.CJ == 2 ? 1 : 0;
-  pr.sK = coarse.CK == 2 ? 1 : 0;
-  pr.nYH = coarse.g.ny;
-  pr.nZH = coarse.g.nz;
-  hipLaunchKernelGGL((k_post2<M, FLUX, RHO>), dim3(f.nblocks), dim3(kBlock), 0, C->stream, lv.g,
-                     A, lv.r, eout, pr, omega, lv.aflag, st, C->work, zscale, f.R, f.TI,
-                     f.ntiles, qf);
-  if (RHO) finalize<kRhoParts>(C, qf ? FIN_RHO_FLEX : FIN_RHO, f.nblocks, st);
-}
-
-template <typename T, bool RHO>
-bool post2(psb_ctx *C, const Level<T> &lv, const T *e, T *eout, const Level<T> &coarse,
-           const T *eH, T cfac, T omega, T zscale, DevState *st, const T *qf = nullptr) {
-  if constexpr (std::is_same<T, float>::value) {
-    FuseShape f;
-    if (!C->fuse || !fuse_shape(lv.g, f)) return false;
-    if (lv.h16() && lv.d)
-      post2_m<RHO, _Float16, true>(C, lv, lv.mat16(), e, eout, coarse, eH, cfac, omega, zscale,
-                                   st, f, qf);
-    else if (lv.h16())
-      post2_m<RHO, _Float16, false>(C, lv, lv.mat16(), e, eout, coarse, eH, cfac, omega, zscale,
-                                    st, f, qf);
-    else if (lv.d)
-      post2_m<RHO, float, true>(C, lv, lv.matflux(), e, eout, coarse, eH, cfac, omega, zscale,
-                                st, f, qf);
-    else
-      post2_m<RHO, float, false>(C, lv, lv.mat(), e, eout, coarse, eH, cfac, omega, zscale, st,
-                                 f, qf);
-    return true;
-  } else {
-    return false;
-  }
-}
-
 template <typename T, int V, int KV, int CI, int CJ, int CK, typename M, bool FLUX>
 void restrict_launch(psb_ctx *C, const Level<T> &f, DMat<M> A, const T *e, Level<T> &cL,
                      T omega, DevState *st) {
@@ -592,6 +544,49 @@ bool pre_restrict(psb_ctx *C, const Level<T> &lv, const T *e, T *eout, Level<T> 
   } else {
     pre_restrict_m<T, T, false>(C, lv, lv.mat(), e, eout, cL, omega, omegaH, st, s);
   }
+  return true;
+}
+
+// the two post-sweeps of level lv in one pass (e and the correction eH of cL
+// to eout); false where the level does not suit it
+template <typename T, bool RHO, typename M, bool FLUX>
+void post_two_m(psb_ctx *C, const Level<T> &lv, DMat<M> A, const T *e, T *eout,
+                const Level<T> &cL, const T *eH, T cfac, T omega, T zscale, DevState *st,
+                const TwoShape &s, const T *qf) {
+  constexpr int V = vmax<T>();
+  auto go = [&](auto ck) {
+    constexpr int CK = decltype(ck)::value;
+    TwoProl<T, V, CK> pr{e, eH, lv.aflag, cfac, lv.g.sI, cL.g.sI, cL.CI >> 1, cL.CJ >> 1, cL.g.nz};
+    hipLaunchKernelGGL((k_post_two<T, V, M, FLUX, CK, RHO>), dim3(s.nblocks), dim3(s.threads),
+                       s.lds * sizeof(T), C->stream, lv.g, A, lv.r, pr, eout, omega, zscale,
+                       lv.aflag, qf, st, C->work, s);
+  };
+  if (cL.CK == 2) go(std::integral_constant<int, 2>());
+  else go(std::integral_constant<int, 1>());
+}
+template <typename T, bool RHO>
+bool post_two(psb_ctx *C, const Level<T> &lv, const T *e, T *eout, const Level<T> &cL,
+              const T *eH, T cfac, T omega, T zscale, DevState *st, const T *qf) {
+  TwoShape s{};
+  if (lv.ae || !two_shape<T>(C, lv.g, s) || s.nblocks > kMaxBlocks) return false;
+  if (std::is_same<T, float>::value && !lv.d) return false;
+  // four coefficient arrays, r, e in, e out; the coarse correction, q, the flags
+  ProbeScope ps(C, RHO ? PSB_K_SWEEP_LAST : PSB_K_SWEEP_PROL, lv.g,
+                4.0 * (lv.h16() ? 2 : sizeof(T)) + 3.0 * sizeof(T) +
+                    (double)sizeof(T) / (cL.CI * cL.CJ * cL.CK) + (RHO && qf ? sizeof(T) : 0) +
+                    (lv.aflag ? 1 : 0));
+  if constexpr (std::is_same<T, float>::value) {
+    if (lv.h16())
+      post_two_m<T, RHO, _Float16, true>(C, lv, lv.mat16(), e, eout, cL, eH, cfac, omega, zscale,
+                                         st, s, qf);
+    else
+      post_two_m<T, RHO, T, true>(C, lv, lv.matflux(), e, eout, cL, eH, cfac, omega, zscale, st,
+                                  s, qf);
+  } else {
+    post_two_m<T, RHO, T, false>(C, lv, lv.mat(), e, eout, cL, eH, cfac, omega, zscale, st, s, qf);
+  }
+  ps.end();
+  if (RHO) finalize<kRhoParts>(C, qf ? FIN_RHO_FLEX : FIN_RHO, s.nblocks, st);
   return true;
 }
 
@@ -1310,11 +1305,12 @@ T *vcycle(psb_ctx *C, Hier<T> &H, int l, DevState *st, int nu1, int nu2, T omega
   const T cfac_l = T((kc ? 1.0 : (double)cfac) * (cL.scale / lv.scale));
   if (nu2 == 2) {  // both post-sweeps in one pass where the level suits it
     const int out = (cur + 2) % 3;
-    const bool done = l == 0 && rho0
-                          ? post2<T, true>(C, lv, lv.e[cur], lv.e[out], cL, zH, cfac_l, omega,
-                                           T(lv.scale), st, H.qf)
-                             : post2<T, false>(C, lv, lv.e[cur], lv.e[out], cL, zH, cfac_l,
-                                               omega, T(1), st);
+    const bool rho = l == 0 && rho0;
+    const bool done =
+        rho ? post_two<T, true>(C, lv, lv.e[cur], lv.e[out], cL, zH, cfac_l, omega, T(lv.scale),
+                                st, H.qf)
+            : post_two<T, false>(C, lv, lv.e[cur], lv.e[out], cL, zH, cfac_l, omega, T(1), st,
+                                 nullptr);
     if (done) return lv.e[out];
   }
   for (int s = 0; s < nu2; s++) {
@@ -1765,7 +1761,6 @@ GKey solve_key(const psb_ctx *C, const psb_stop *p, int body, const void *x, con
   k.nu1 = p->ac_pre;
   k.nu2 = p->ac_post;
   k.kmask = C->kmask;
-  k.fuse = C->fuse;
   k.cg16 = C->cg_half;
   k.half = body == 0 || body >= 3 ? 0 : (C->h32.L.empty() ? 0 : C->h32.L[0].use16);
   k.flex = C->flex;
@@ -2625,7 +2620,6 @@ int solve_device(psb_ctx *C, double *x, const double *b, const psb_stop *p, psb_
         return PSB_EINVAL;
       ensure_rule(C, p->ac_coarsen);
       C->cg_half = false;
-      C->fuse = false;
       C->kmask = 0;
       C->flex = false;
       C->ac_omega = p->ac_omega;
@@ -2644,7 +2638,6 @@ int solve_device(psb_ctx *C, double *x, const double *b, const psb_stop *p, psb_
     // settings of this solve, read while its graph is captured (the graph
     // cache keys on them: no setting change drops a graph)
     C->cg_half = p->precision == PSB_MIXED && p->ac_store == 2;
-    C->fuse = p->ac_fuse != 0;
     C->kmask = p->ac_kcycle;
     C->flex_req = p->ac_flexible;  // resolved against the hierarchy (set_flex)
     C->ac_omega = p->ac_omega;
@@ -3289,7 +3282,7 @@ int psb_time_kernel(psb_ctx *C, int kernel, int reps, double *avg_ms, double *by
       // or FP16), e and r in, e out
       *bytes = N * (4 * (lv.h16() ? 2 : 4) + 3 * 4);
     } else if (kernel == 4 || kernel == 5) {
-      // the two post-sweeps of the fine level: 4 in one pass (k_post2), 5 as
+      // the two post-sweeps of the fine level: 4 in one pass (k_post_two), 5 as
       // two kernels; both as the last mixed solve's hierarchy stores the level
       build_hier32(C);
       Level<float> lv = C->h32.L[0];
@@ -3302,11 +3295,8 @@ int psb_time_kernel(psb_ctx *C, int kernel, int reps, double *avg_ms, double *by
       HIPCHK(hipMemcpyAsync(C->st32, &h, sizeof(h), hipMemcpyHostToDevice, stream));
       const bool fused = kernel == 4;
       f = [=]() {
-        const bool keep = C->fuse;
-        C->fuse = true;  // time the fused pass whatever the last solve selected
-        const bool done = fused && post2<float, false>(C, lv, lv.e[0], lv.e[2], cL, cL.e[0], 2.0f,
-                                                       0.9f, 1.0f, C->st32);
-        C->fuse = keep;
+        const bool done = fused && post_two<float, false>(C, lv, lv.e[0], lv.e[2], cL, cL.e[0],
+                                                          2.0f, 0.9f, 1.0f, C->st32, nullptr);
         if (done) return;
         jacobi<float, false>(C, lv, lv.e[0], lv.e[1], &cL, cL.e[0], 2.0f, 0.9f, C->st32);
         jacobi<float, false>(C, lv, lv.e[1], lv.e[2], nullptr, nullptr, 0.0f, 0.9f, C->st32);

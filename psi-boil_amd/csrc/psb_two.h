@@ -1,10 +1,11 @@
 // psb_two.h -- two stencil stages of a level in one pass over it.
 //
-// The last pre-sweep and the restriction both read the level's matrix and
-// right-hand side: as two kernels they stream 37.5 bytes a cell (FP16 smoother
-// copy), 107 (FP64); in one pass 21.5 and 59.  Here a block marches through the i
-// planes with both stages in flight: stage 1 forms plane i of the swept
-// correction while stage 2 works on plane i - 1 of it.
+// The last pre-sweep and the restriction, and the two post-sweeps, each read
+// the level's matrix and right-hand side: as two kernels they stream 37.5 and
+// 44.5 bytes a cell (FP16 smoother copy), 107 and 121 (FP64); in one pass 21.5
+// and 24.5, 59 and 65.  Here a block marches through the i planes with both
+// stages in flight: stage 1 forms plane i of the swept correction while stage 2
+// works on plane i - 1 of it.
 //   * A thread owns one cell vector of a (j, k) tile.  Two planes of the
 //     operand of stage 1 (with a halo row below and above) and of the swept
 //     correction are in LDS, and one barrier per plane orders everything.
@@ -15,12 +16,15 @@
 //     the others may hold anything.
 //   * Matrix, right-hand side and operand of the next plane are loaded a plane
 //     ahead; a plane's w couplings are the plane before's e.
-// What bounds it: at 256^3 (FP16 copy) 386 MB of HBM traffic (1.07 of what it
-// must move) at 4.4 TB/s with the vector units half busy.  Measured, us, this
-// pass against the two kernels:
-//   FP16 copy: 256^3 87 / 78 + 67, 128^3 18 / 11.5 + 9.3, 32^3 7.1 / 4.5 + 5.5
-//   FP64:      256^3 216 / 399, 128^3 31 / 25 + 21, 32^3 6.7 / 3.9 + 4.9
-// The arithmetic is the separate kernels' (gather_c): bit-identical.
+// What bounds it: at 256^3 (FP16 copy) the first pair takes 386 MB of HBM
+// traffic (1.07 of what it must move) at 4.4 TB/s with the vector units half
+// busy.  Measured, us, one pass against two kernels:
+//   first pair, FP16 copy: 256^3 87 / 78 + 67, 128^3 18 / 11.5 + 9.3, 32^3 7.1 / 4.5 + 5.5
+//   first pair, FP64:      256^3 216 / 399, 128^3 31 / 25 + 21, 32^3 6.7 / 3.9 + 4.9
+//   post-sweeps, FP16 copy: 256^3 100 / 76 + 81, 128^3 18.6 / 11.5 + 11.7, 32^3 8.2 / 4.5 + 4.7
+//   post-sweeps, FP64:      256^3 324 / 195 + 214, 128^3 25 / 25 + 21, 32^3 6.4 / 4.6 + 4.6
+// The arithmetic is the separate kernels' (gather_c), so that the results are
+// bit-identical; only the rho partials are summed over other blocks.
 #pragma once
 
 #include "psb_march.h"
@@ -199,7 +203,8 @@ __device__ __forceinline__ TwoAt two_at(const Grid &g, const TwoShape &s) {
 }
 
 // stage 1's operand, loaded apart from the arithmetic that forms it (which
-// would wait for the loads where it stands)
+// would wait for the loads where it stands): an array, or with the
+// prolongation e + cfac * eH[parent] (ProlX; CK the coarsening along k)
 template <typename T, int V>
 struct TwoArr {
   const T *e;
@@ -216,6 +221,43 @@ struct TwoArr {
   }
   __device__ __forceinline__ VecN<T, V> form(const Raw &x) const { return x; }
 };
+template <typename T, int V, int CK>
+struct TwoProl {
+  const T *e, *eH;
+  const uint8_t *af;
+  T cfac;
+  int sI, sIH, pI, pJ, nZH;  // plane sizes, coarsening shifts along i and j
+  struct At {
+    uint32_t o, h, f;
+  };
+  struct Raw {
+    VecN<T, V> E;
+    VecN<T, V / CK> H;
+    uint32_t f;
+  };
+  __device__ __forceinline__ At place(int j, int k, int nz) const {
+    const uint32_t P = (uint32_t)(j * nz + k);
+    return At{P * (uint32_t)sizeof(T), (uint32_t)((j >> pJ) * nZH + k / CK) * (uint32_t)sizeof(T),
+              P};
+  }
+  __device__ __forceinline__ Raw load(int i, const At &a) const {
+    Raw x;
+    x.E = ldo<T, V>(e + (size_t)i * sI, a.o);
+    x.H = ldo<T, V / CK>(eH + (size_t)(i >> pI) * sIH, a.h);
+    x.f = af ? ldflags<V>(af + (size_t)i * sI, a.f) : 0xffffffffu;
+    return x;
+  }
+  __device__ __forceinline__ VecN<T, V> form(const Raw &x) const {
+    VecN<T, V> o;
+#pragma unroll
+    for (int u = 0; u < V; u++) {
+      const T v = x.E.v[u] + cfac * x.H.v[u / CK];
+      o.v[u] = !af || flag_on(x.f, u) ? v : x.E.v[u];
+    }
+    return o;
+  }
+};
+
 // the swept correction of plane i in the step after the one that formed it
 template <typename T, int V>
 __device__ __forceinline__ VecN<T, V> two_swept(const TwoShape &s, const TwoAt &a, const T *lds,
@@ -425,6 +467,77 @@ __global__ __launch_bounds__(kTwoThreads) void k_pre_restrict(
   load_c(a.i1);
   Qd = (a.i1 - 1) >> 1;
   store();
+}
+
+// the two post-sweeps of a level, the prolongation of eH fused into the first
+// (as k_jacobi with PROL, then without); RHO: the finest level, whose second
+// sweep leaves z times zscale and the rho partials (rho_accq), one set per
+// block
+template <typename T, int V, typename M, bool FLUX, int CK, bool RHO>
+__global__ __launch_bounds__(kTwoThreads) void k_post_two(Grid g, DMat<M> A, const T *r,
+                                                          TwoProl<T, V, CK> pr, T *eout, T omega,
+                                                          T zscale, const uint8_t *af,
+                                                          const T *qf, const DevState *st, Work w,
+                                                          TwoShape s) {
+  if (skip_done(st, g.N)) return;
+  extern __shared__ __align__(16) char two_lds[];
+  T *const lds = reinterpret_cast<T *>(two_lds);
+  const TwoAt a = two_at<V>(g, s);
+  const uint32_t oT = a.P * (uint32_t)sizeof(T);
+  double acc[kRhoParts] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  int count = 0;   // active cells (an integer takes half the registers)
+  VecN<T, V> z{};  // a plane's result, stored a step later
+  struct Q {
+    VecN<T, V> q;
+    uint32_t f;
+  };
+  auto put = [&](int i) {
+    if (a.out) sto<T, V>(eout + (size_t)i * g.sI, oT, z);
+  };
+  two_march<T, V, M, FLUX>(
+      g, A, r, pr, omega, s, a, lds, [&](int i) {
+        if (i > a.i0) put(i - 1);
+      },
+      [&](int i) {
+        Q o{};
+        if constexpr (RHO) {
+          o.q = ldo<T, V>((qf ? qf : r) + (size_t)i * g.sI, oT);
+          o.f = af ? ldflags<V>(af + (size_t)i * g.sI, a.P) : 0xffffffffu;
+        }
+        return o;
+      },
+      [&](int, const Gath<T, V> &G, const VecN<T, V> &R, const TwoRow<T, V> &row,
+          const VecN<T, V> &E, const Q &o) {
+        z = row.template sweep<FLUX>(E, R, G, omega);
+        if constexpr (RHO) {
+#pragma unroll
+          for (int u = 0; u < V; u++) {
+            z.v[u] = zscale * z.v[u];
+            const bool on = !af || flag_on(o.f, u);
+            rho_accq<T, false>(acc, R.v[u], z.v[u], qf != nullptr, o.q.v[u], on);
+            count += on ? 1 : 0;
+          }
+        }
+      },
+      [](int) {});
+  put(a.i1 - 1);
+  if constexpr (RHO) {
+    acc[3] = (double)count;
+    // one partial per block: wave sums, then the waves in turn
+    __shared__ double sm[kTwoThreads / 64][kRhoParts];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (int)blockDim.x >> 6;
+#pragma unroll
+    for (int q = 0; q < kRhoParts; q++) {
+      const double v = wave_sum(acc[q]);
+      if (lane == 0) sm[wid][q] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x < kRhoParts) {
+      double t = 0.0;
+      for (int q = 0; q < nw; q++) t += sm[q][threadIdx.x];
+      w.partial[(size_t)blockIdx.x * kRhoParts + threadIdx.x] = t;
+    }
+  }
 }
 
 }  // namespace psb
