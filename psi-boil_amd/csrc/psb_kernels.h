@@ -457,6 +457,76 @@ __device__ inline double fold_pq(const Fold &f, DevState *st, double rho) {
   return alpha;
 }
 
+// BiCGS's three steps in the kernels that use their results.  FIN_BI3 in the
+// next iteration's p/v step (as fold_xr_diag): returns whether the solve has
+// stopped, else beta and omega.
+__device__ inline bool fold_bi3(const Fold &f, const StopIn &s, const DevState *in, double &beta,
+                                double &omega) {
+  const double alpha = in->alpha, ss = in->rv_ss;
+  omega = in->omega;
+  if (blockIdx.x == 0)
+    for (int q = threadIdx.x; q < kStateWords; q += kBlock)
+      reinterpret_cast<uint64_t *>(f.out)[q] = reinterpret_cast<const uint64_t *>(in)[q];
+  double tot[3];
+  fin_sum<3>(0, f.nprev, f.prev, tot);  // its barriers order the copy before the step's fields
+  if (s.done) return true;
+  const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+  if (sqrt(ss) < s.res_tol) {  // bicgs.cpp:134-138
+    if (writer) {
+      f.out->done = 1;
+      f.out->converged = 0;
+      f.out->reason = 5;
+      f.out->report_iters = s.iter + 1;
+    }
+    return true;
+  }
+  const double res = s.norm == 0 ? ref_norm(&s, tot[0]) : sqrt(tot[1]);
+  const StopOut o =
+      krylov_decide(s, in->stale, res, omega >= -s.res_tol && omega <= s.res_tol);
+  const bool breakdown = sqrt(fabs(tot[2])) < s.res_tol;  // bicgs.cpp:84-89
+  beta = (tot[2] / s.rho) * (alpha / omega);              // bicgs.cpp:102
+  if (writer) {
+    f.out->rsq = tot[1];
+    krylov_put(f.out, s, o, res);
+    if (!o.done && breakdown) {
+      f.out->done = 1;
+      f.out->reason = 4;
+      f.out->report_iters = s.iter + 2;
+    } else if (!o.done) {
+      f.out->beta = beta;
+      f.out->rho = tot[2];
+    }
+  }
+  return o.done || breakdown;
+}
+
+// FIN_BI1: alpha (later kernels read the state's)
+__device__ inline double fold_bi1(const Fold &f, DevState *st) {
+  const double rho = st->rho;
+  double tot[1];
+  fin_sum<1>(0, f.nprev, f.prev, tot);
+  const double alpha = rho / tot[0];  // bicgs.cpp:122-123
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->rv = tot[0];
+    st->alpha = alpha;
+  }
+  return alpha;
+}
+
+// FIN_BI2: s.s and omega
+__device__ inline void fold_bi2(const Fold &f, DevState *st, double &ss, double &omega) {
+  double tot[3];
+  fin_sum<3>(0, f.nprev, f.prev, tot);
+  ss = tot[0];
+  omega = tot[1] / tot[2];  // bicgs.cpp:155-157
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->rv_ss = ss;
+    st->rv_ts = tot[1];
+    st->rv_tt = tot[2];
+    st->omega = omega;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // y = A x   (Scalar::operator=(A_x), scalar_operators.cpp:49-72)
 // ---------------------------------------------------------------------------
@@ -1205,11 +1275,18 @@ struct BiPX {
 template <typename T, int V, bool SYM>
 __global__ __launch_bounds__(kBlock) void k_bi1(Grid g, DMat<T> A, const T *r, const T *rt,
                                                 const T *pold, const T *vold, T *pnew,
-                                                T *vnew, DevState *st, Work w) {
-  if (st->done) return;
-  const bool first = st->iter == 0;
-  const T beta = first ? T(0) : (T)st->beta;
-  const T bo = first ? T(0) : (T)(st->beta * st->omega);
+                                                T *vnew, const DevState *st, Work w, Fold f) {
+  double be, om;
+  if (f.nprev) {
+    if (fold_bi3(f, StopIn(st), st, be, om)) return;
+  } else {
+    if (st->done) return;
+    be = st->beta;
+    om = st->omega;
+  }
+  const bool first = !f.nprev && st->iter == 0;
+  const T beta = first ? T(0) : (T)be;
+  const T bo = first ? T(0) : (T)(be * om);
   BiPX<T, V> X{r, pold, vold, A.c, beta, bo};
   double acc[1] = {0.0};
   PSB_TILE_BEGIN(g, V)
@@ -1246,9 +1323,9 @@ struct BiSX {
 
 template <typename T, int V, bool SYM>
 __global__ __launch_bounds__(kBlock) void k_bi2(Grid g, DMat<T> A, const T *r, const T *v,
-                                                T *s, T *t, DevState *st, Work w) {
+                                                T *s, T *t, DevState *st, Work w, Fold f) {
   if (st->done) return;
-  BiSX<T, V> X{r, v, A.c, (T)st->alpha};
+  BiSX<T, V> X{r, v, A.c, (T)(f.nprev ? fold_bi1(f, st) : st->alpha)};
   double acc[3] = {0.0, 0.0, 0.0};  // ss, ts, tt
   PSB_TILE_BEGIN(g, V)
   Gath<T, V> G = gather<T, V, SYM>(g, A, X, P, i, j, k);
@@ -1271,10 +1348,17 @@ __global__ __launch_bounds__(kBlock) void k_bi2(Grid g, DMat<T> A, const T *r, c
 template <typename T, int V>
 __global__ __launch_bounds__(kBlock) void k_bi3(Grid g, const T *c, Metric m, const T *p,
                                                 const T *s, const T *t, const T *rt, T *x,
-                                                T *r, DevState *st, Work w) {
+                                                T *r, DevState *st, Work w, Fold f) {
   if (st->done) return;
-  const bool small_s = sqrt(st->rv_ss) < st->res_tol;
-  const T alpha = (T)st->alpha, omega = (T)st->omega;
+  double ss, om;
+  if (f.nprev) {
+    fold_bi2(f, st, ss, om);
+  } else {
+    ss = st->rv_ss;
+    om = st->omega;
+  }
+  const bool small_s = sqrt(ss) < st->res_tol;
+  const T alpha = (T)st->alpha, omega = (T)om;
   double acc[3] = {0.0, 0.0, 0.0};  // voldiv, r^2, rho_next
   PSB_TILE_BEGIN(g, V)
   VecN<T, V> X = ldv<T, V>(x + P), Pp = ldv<T, V>(p + P), C = ldv<T, V>(c + P);
