@@ -30,6 +30,7 @@
 #include "psb_lds.h"
 #include "psb_tail.h"
 #include "psb_two.h"
+#include "psb_dense.h"
 #include "psb_internal.h"
 
 // FP32 levels evaluate the stencil in flux form (set to 0 for the plain form)
@@ -656,8 +657,7 @@ std::vector<double> dense_pinv(bool project, int nx, int ny, int nz, const std::
   }
   // columns of the inverse: two banded triangular solves each (the forward
   // one starts at the column's own row: y is zero above it), independent,
-  // on the host's threads (the coarsest level of a stretched grid can hold
-  // 12^3 = 1728 cells)
+  // on the host's threads
   std::vector<double> B((size_t)m * m, 0.0);
   auto columns = [&](int c0, int c1) {
     std::vector<double> y(m);
@@ -853,6 +853,46 @@ std::vector<double> dense_inv(int nx, int ny, int nz, const std::vector<double> 
   return G;
 }
 
+// dense_pinv's G of level cl by the kernels of psb_dense.h, where the band fits
+// them; false elsewhere (and for 7 arrays)
+bool device_pinv(psb_ctx *C, const Level<double> &cl, double *G) {
+  const Grid &g = cl.g;
+  const int m = g.N, bw = g.nx > 1 ? g.ny * g.nz : (g.ny > 1 ? g.nz : 1), n = bw + 1;
+  if (!C->dense || cl.ae || bw > kBandMax || m > kBandMaxCells) return false;
+  Arena &ar = C->harena;
+  BandArgs A{g.nx, g.ny, g.nz, bw, cl.c, cl.w, cl.s, cl.b, cl.aflag,
+             ar.alloc<double>((size_t)m * n), ar.alloc<double>((size_t)m * n)};
+  double *Bt = ar.alloc<double>((size_t)m * m), *cm = ar.alloc<double>(m),
+         *rm = ar.alloc<double>(m + 1);
+  auto chol = [&](auto u) {
+    hipLaunchKernelGGL((k_band_chol<decltype(u)::value>), dim3(1), dim3(kBandThreads),
+                       (size_t)n * (n + 1) / 2 * sizeof(double), C->stream, A);
+  };
+  const int per = (bw * n / 2 + kBandThreads - 1) / kBandThreads;  // products per thread
+  if (per <= 3) chol(std::integral_constant<int, 3>());
+  else if (per <= 6) chol(std::integral_constant<int, 6>());
+  else if (per <= 11) chol(std::integral_constant<int, 11>());
+  else chol(std::integral_constant<int, 19>());
+  auto inverse = [&](auto q) {
+    hipLaunchKernelGGL((k_band_inverse<decltype(q)::value>), dim3(m), dim3(64),
+                       (size_t)m * sizeof(double), C->stream, A, Bt, cm);
+  };
+  if (n <= 64) inverse(std::integral_constant<int, 1>());
+  else if (n <= 128) inverse(std::integral_constant<int, 2>());
+  else inverse(std::integral_constant<int, 4>());
+  const int nt = (m + 15) / 16;
+  hipLaunchKernelGGL(k_band_turn, dim3(nt * nt), dim3(kBlock), 0, C->stream, m, Bt, G);
+  if (C->singular) {
+    hipLaunchKernelGGL(k_band_rows, dim3((m + 63) / 64), dim3(64), 0, C->stream, m, Bt, rm);
+    hipLaunchKernelGGL(k_band_total, dim3(1), dim3(1024), 0, C->stream, (long long)m * m, G,
+                       rm + m);
+    hipLaunchKernelGGL(k_band_project, dim3(m), dim3(kBlock), 0, C->stream, m, cl.aflag, rm, cm,
+                       rm + m, G);
+  }
+  HIPCHK(hipGetLastError());
+  return true;
+}
+
 void build_hier64(psb_ctx *C) {
   Hier<double> &H = C->h64;
   if (H.built) return;
@@ -900,6 +940,13 @@ void build_hier64(psb_ctx *C) {
   // coarsest dense operator
   Level<double> &cl = H.L[nl - 1];
   const int m = cl.g.N;
+  H.m = m;
+  H.G = C->harena.alloc<double>((size_t)m * m);
+  if (device_pinv(C, cl, H.G)) {
+    HIPCHK(hipStreamSynchronize(stream));
+    H.built = true;
+    return;
+  }
   std::vector<double> c(m), w(m), s(m), b(m);
   std::vector<uint8_t> act(m, 1);
   HIPCHK(hipMemcpyAsync(c.data(), cl.c, m * 8, hipMemcpyDeviceToHost, stream));
@@ -918,8 +965,6 @@ void build_hier64(psb_ctx *C) {
   std::vector<double> G = cl.ae ? dense_inv(cl.g.nx, cl.g.ny, cl.g.nz, c, w, s, b, e, n, t, act)
                                 : dense_pinv(C->singular, cl.g.nx, cl.g.ny, cl.g.nz, c, w, s, b,
                                              act);
-  H.m = m;
-  H.G = C->harena.alloc<double>((size_t)m * m);
   HIPCHK(hipMemcpyAsync(H.G, G.data(), (size_t)m * m * 8, hipMemcpyHostToDevice, stream));
   HIPCHK(hipStreamSynchronize(stream));
   H.built = true;
@@ -2804,6 +2849,7 @@ int psb_create(psb_ctx **out, const psb_layout *L) {
     if (std::getenv("PSB_NO_TAIL")) C->tail = false;
     if (std::getenv("PSB_NO_FOLD")) C->fold = false;
     if (std::getenv("PSB_NO_TWO")) C->two = false;
+    if (std::getenv("PSB_NO_DENSE")) C->dense = false;
     if (std::getenv("PSB_NO_LDS")) {
       C->lds32 = C->lds64 = 0;
     } else if (const char *m = std::getenv("PSB_LDS_MASK")) {

@@ -289,6 +289,9 @@ struct psb_ctx {
   // two stages of a level in one pass (psb_two.h; PSB_NO_TWO set: one kernel
   // each, for comparisons)
   bool two = true;
+  // the coarsest level's dense operator formed on the device (psb_dense.h;
+  // PSB_NO_DENSE set: on the host, for comparisons)
+  bool dense = true;
   // the pressure's boundary conditions for the device assembly (all Neumann,
   // value 0: walls) and the boundary source it formed (NULL: none)
   psb_bnd bnd{};
