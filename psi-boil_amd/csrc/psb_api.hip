@@ -489,7 +489,8 @@ bool two_shape(const psb_ctx *C, const Grid &g, TwoShape &s) {
     for (int R = 2; (R + 2) * KT <= kTwoThreads; R += 2) {
       const size_t lds = (size_t)(2 * (R + 4) + 2 * (R + 2) + R) * KT * V;
       if (lds * sizeof(T) > 150 * 1024) break;
-      const int waves = ((R + 2) * KT + 63) / 64, per_cu = std::max(1, 12 / waves);
+      // (blocks share a compute unit where their waves spread evenly over its SIMDs)
+      const int waves = ((R + 2) * KT + 63) / 64, per_cu = waves > 4 ? 1 : 12 / (waves > 2 ? 4 : 2);
       const long long nt = (long long)((g.ny + R - 1) / R) * ntk;
       for (int TI = 2; TI < g.nx + 2; TI += 2) {
         const long long nb = nt * ((g.nx + TI - 1) / TI);

@@ -54,6 +54,13 @@ struct SegList {
   bool empty() const { return segs.empty(); }
 };
 
+// the two-stage passes of a level (empty: one kernel per stage)
+struct TwoList {
+  SegList L;
+  int threads = 0, CK = 0;
+  size_t lds = 0;  // bytes
+};
+
 }  // namespace
 
 struct psb_batch {
@@ -83,6 +90,7 @@ struct psb_batch {
   SegList fine64L;                              // all systems, fine level (FP64 vectors)
   std::vector<SegList> smoothL;                 // [l]: systems with l < last
   std::vector<std::vector<std::pair<int, SegList>>> restrictL;  // [l]: (CI,CJ,CK) groups
+  std::vector<TwoList> twoL;                    // [l]: smoothL's systems, two-stage passes
   std::vector<SegList> gemvL;                   // [l]: systems with last == l
   Graph graph;
   double omega = 0, cfac = 0;
@@ -160,6 +168,76 @@ BSeg level_seg(const psb_batch *B, int l, int s, long long nwork) {
   return make_seg(s, nwork, B->vpt[l][s]);
 }
 
+// The two-stage passes' tile for a level of one system, slabs of TI planes: rows
+// whole where six output rows fit kBatchTwo threads (three blocks to a compute
+// unit, one wave of each on every SIMD, so that one computes while another waits
+// at its barrier) or a block of kTwoThreads, else split along k; the rows shared
+// out evenly.  Measured, 96 systems of 32 to 128 cells a side, us, level 0 / 1:
+// 256 threads 162 / 28, 384 (one block to a unit) 214 / 47, 768 214 / 49, 128
+// (rows of 128 cells in blocks of 768) 396 / 27.
+constexpr int kBatchTwo = 256;
+void batch_two_shape(const Grid &g, int TI, TwoShape &s) {
+  const int nv = g.nz / 4;
+  int KO = nv, KT = nv, cap = kBatchTwo;
+  if ((cap / KT - 2) < 6) cap = kTwoThreads;
+  if ((cap / KT - 2) < 6) {
+    KO = 32;
+    KT = KO + 2;
+  }
+  int R = (cap / KT - 2) & ~1;
+  const int ntj = (g.ny + R - 1) / R;
+  R = (((g.ny + ntj - 1) / ntj) + 1) & ~1;
+  s.RT = R + 2;
+  s.KT = KT;
+  s.KO = KO;
+  s.ntj = ntj;
+  s.ntk = (nv + KO - 1) / KO;
+  s.TI = TI;
+  s.nblocks = s.ntj * s.ntk * ((g.nx + TI - 1) / TI);
+  s.threads = (s.RT * KT + 63) / 64 * 64;
+  s.lds = (size_t)(2 * (R + 4) + 2 * (R + 2) + R) * KT * 4;
+}
+
+// level l's list where every system that smooths there has 4-wide vectors and
+// halves x and y (and all or none z).  Depth of the slabs: the rounds of blocks,
+// three to a compute unit and one more that is partly empty, times the steps of
+// one (measured as above, 32 / 16 / 8 / 4 planes: level 0 194 / 162 us, level 1
+// 43 / 28 / 28 / 32)
+void build_two(psb_batch *B, int l) {
+  TwoList &W = B->twoL[l];
+  const std::vector<BSeg> &who = B->smoothL[l].segs;
+  if (who.empty() || B->Vl[l] != 4) return;
+  const int sK = B->lev[l + 1][who[0].sys].sK;
+  for (const BSeg &q : who) {
+    const BLev<float> &H = B->lev[l + 1][q.sys];
+    if (!B->sys[q.sys]->two || !H.sI || !H.sJ || H.sK != sK) return;
+  }
+  long long least = 0;
+  int depth = 2;
+  for (int TI = 32; TI >= 2; TI /= 2) {
+    long long blocks = 0;
+    TwoShape s;
+    for (const BSeg &q : who) {
+      batch_two_shape(B->lev[l][q.sys].g, TI, s);
+      blocks += s.nblocks;
+    }
+    const long long cost = (blocks + 768) * (TI + 3);
+    if (least == 0 || cost < least) {
+      least = cost;
+      depth = TI;
+    }
+  }
+  for (const BSeg &q : who) batch_two_shape(B->lev[l][q.sys].g, depth, B->lev[l][q.sys].two);
+  W.CK = sK ? 2 : 1;
+  for (const BSeg &q : who) {
+    const TwoShape &s = B->lev[l][q.sys].two;
+    W.threads = std::max(W.threads, s.threads);
+    W.lds = std::max(W.lds, s.lds * sizeof(float));
+    W.L.segs.push_back(BSeg{q.sys, 0, round8(s.nblocks), 0});
+  }
+  upload_list(B, W.L);
+}
+
 // launch lists for the current per-(level, system) tiles
 void build_lists(psb_batch *B) {
   const int ns = B->nsys;
@@ -175,6 +253,7 @@ void build_lists(psb_batch *B) {
   B->smoothL.assign(B->nlev, SegList());
   B->gemvL.assign(B->nlev, SegList());
   B->restrictL.assign(B->nlev, {});
+  B->twoL.assign(B->nlev, TwoList());
   for (int l = 0; l < B->nlev; l++) {
     std::map<int, SegList> groups;
     for (int s = 0; s < ns; s++) {
@@ -191,6 +270,7 @@ void build_lists(psb_batch *B) {
     }
     if (l == 0) B->smoothL[0] = B->fineL;  // level 0: the fine partition (RHO partials)
     else upload_list(B, B->smoothL[l]);
+    if (l + 1 < B->nlev) build_two(B, l);
     upload_list(B, B->gemvL[l]);
     for (auto &kv : groups) {
       upload_list(B, kv.second);
@@ -199,6 +279,7 @@ void build_lists(psb_batch *B) {
   }
   int most = B->fineL.nblocks;
   for (const SegList &L : B->smoothL) most = std::max(most, L.nblocks);
+  for (const TwoList &W : B->twoL) most = std::max(most, W.L.nblocks);
   B->partial = B->arena.alloc<double>((size_t)most * kMaxPartials);
 }
 
@@ -281,10 +362,38 @@ void l_restrict(psb_batch *B, int l, int cur) {
   }
 }
 
+// level l's last pre-sweep and restriction, or its two post-sweeps, in one pass
+bool l_pre_restrict(psb_batch *B, int l, int cur, int nxt) {
+  const TwoList &W = B->twoL[l];
+  if (W.L.empty()) return false;
+  auto go = [&](auto ck) {
+    hipLaunchKernelGGL((kb_pre_restrict<decltype(ck)::value>), dim3(W.L.nblocks),
+                       dim3(W.threads), W.lds, B->stream, W.L.d_segs, W.L.d_bmap, B->d_fine,
+                       B->d_lev[l], B->d_lev[l + 1], cur, nxt, (float)B->omega);
+  };
+  if (W.CK == 2) go(std::integral_constant<int, 2>());
+  else go(std::integral_constant<int, 1>());
+  return true;
+}
+template <bool RHO>
+bool l_post_two(psb_batch *B, int l, int cur, int nxt, int outH) {
+  const TwoList &W = B->twoL[l];
+  if (W.L.empty()) return false;
+  auto go = [&](auto ck) {
+    hipLaunchKernelGGL((kb_post_two<decltype(ck)::value, RHO>), dim3(W.L.nblocks),
+                       dim3(W.threads), W.lds, B->stream, W.L.d_segs, W.L.d_bmap, B->d_fine,
+                       B->d_lev[l], B->d_lev[l + 1], cur, nxt, outH, (float)B->cfac,
+                       (float)B->omega, Work{B->partial}, RHO && B->flex);
+  };
+  if (W.CK == 2) go(std::integral_constant<int, 2>());
+  else go(std::integral_constant<int, 1>());
+  return true;
+}
+
+// (L: the list whose blocks left the partials)
 template <int NR>
-void l_finalize(psb_batch *B, int op) {
-  hipLaunchKernelGGL((kb_finalize<NR>), dim3(B->nsys), dim3(kBlock), 0, B->stream, op,
-                     B->fineL.d_segs, B->d_fine, B->partial, B->flags);
+void l_finalize(psb_batch *B, int op, const SegList &L) {
+  hipLaunchKernelGGL((kb_finalize<NR>), dim3(B->nsys), dim3(kBlock), 0, B->stream, op, L.d_segs, B->d_fine, B->partial, B->flags);
 }
 
 void l_ru_resid(psb_batch *B, bool gated, int op) {
@@ -296,7 +405,7 @@ void l_ru_resid(psb_batch *B, bool gated, int op) {
   else
     hipLaunchKernelGGL((kb_ru_resid<1>), dim3(L.nblocks), dim3(kBlock), 0, B->stream, L.d_segs,
                        L.d_bmap, B->d_fine, B->d_lev[0], (float)B->omega, gated, w);
-  l_finalize<4>(B, op);
+  l_finalize<4>(B, op, B->fineL);
 }
 
 void l_ru_xupdate(psb_batch *B, bool gated) {
@@ -356,14 +465,19 @@ void b_cycle(psb_batch *B, int l, int nu1, int nu2) {
                        G.d_bmap, B->d_fine, B->d_lev[l], out);
   if (B->smoothL[l].empty()) return;
   int cur = 0;
+  bool restricted = false;
   for (int s = 1; s < nu1; s++) {
     const int nxt = (cur + 1) % 3;
-    l_jacobi<false, false>(B, l, cur, nxt, 0);
+    restricted = s == nu1 - 1 && l_pre_restrict(B, l, cur, nxt);
+    if (!restricted) l_jacobi<false, false>(B, l, cur, nxt, 0);
     cur = nxt;
   }
-  l_restrict(B, l, cur);
+  if (!restricted) l_restrict(B, l, cur);
   if ((B->kmask >> (l + 1)) & 1) b_kstep(B, l + 1, nu1, nu2);
   else b_cycle(B, l + 1, nu1, nu2);
+  if (nu2 == 2 && (l == 0 ? l_post_two<true>(B, l, cur, (cur + 2) % 3, out)
+                          : l_post_two<false>(B, l, cur, (cur + 2) % 3, out)))
+    return;
   for (int s = 0; s < nu2; s++) {
     const int nxt = (cur + 1) % 3;
     const bool last = (s == nu2 - 1) && l == 0;
@@ -379,7 +493,8 @@ void b_cycle(psb_batch *B, int l, int nu1, int nu2) {
 // and the rho step
 void b_vcycle(psb_batch *B, int nu1, int nu2) {
   b_cycle(B, 0, nu1, nu2);
-  l_finalize<kRhoParts>(B, B->flex ? FIN_RHO_FLEX : FIN_RHO);
+  const bool two = nu2 == 2 && !B->twoL[0].L.empty();
+  l_finalize<kRhoParts>(B, B->flex ? FIN_RHO_FLEX : FIN_RHO, two ? B->twoL[0].L : B->fineL);
 }
 
 void b_iteration(psb_batch *B, int par, int nu1, int nu2) {
@@ -394,7 +509,7 @@ void b_iteration(psb_batch *B, int par, int nu1, int nu2) {
     hipLaunchKernelGGL((kb_cg_pq<1>), dim3(L.nblocks), dim3(kBlock), 0, B->stream, L.d_segs,
                        L.d_bmap, B->d_fine, B->d_lev[0], out, par, w);
   }
-  l_finalize<1>(B, FIN_PQ);
+  l_finalize<1>(B, FIN_PQ, B->fineL);
   if (B->V == 4) {
     hipLaunchKernelGGL((kb_cg_xr<4>), dim3(L.nblocks), dim3(kBlock), 0, B->stream, L.d_segs,
                        L.d_bmap, B->d_fine, B->d_lev[0], par, (float)B->omega, w);
@@ -402,7 +517,7 @@ void b_iteration(psb_batch *B, int par, int nu1, int nu2) {
     hipLaunchKernelGGL((kb_cg_xr<1>), dim3(L.nblocks), dim3(kBlock), 0, B->stream, L.d_segs,
                        L.d_bmap, B->d_fine, B->d_lev[0], par, (float)B->omega, w);
   }
-  l_finalize<3>(B, FIN_XR_RU);
+  l_finalize<3>(B, FIN_XR_RU, B->fineL);
   l_ru_xupdate(B, true);
   l_ru_resid(B, true, FIN_RU);
 }

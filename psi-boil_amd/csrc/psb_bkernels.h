@@ -8,6 +8,7 @@
 
 #include "psb_kernels.h"
 #include "psb_march.h"
+#include "psb_two.h"
 
 namespace psb {
 
@@ -25,6 +26,7 @@ struct BLev {
   const double *G;    // coarsest level: dense projected pseudo-inverse
   int TI, ntiles;     // TI > 0: the Jacobi sweeps (and on level 0 the CG p/q
                       // step) march, slabs of TI planes, ntiles tiles a plane
+  TwoShape two;       // tiles of the two-stage passes (psb_two.h)
   int kcyc;           // this level's correction is the K-cycle's (in kz)
   T *kc, *kv, *kz;    // K-cycle: first cycle's output, A of it, the correction
   double *kst;        // K-cycle scalars rho1, alpha1, a, alpha2
@@ -104,6 +106,42 @@ __global__ __launch_bounds__(kBlock) void kb_restrict(const BSeg *segs, const ui
   const BLev<T> &H = levH[sg_.sys];
   restrict_body<T, V, KV, true, CI, CJ, CK, T, true>(sp, L.g, L.matflux(), L.r, L.e[cur], L.af,
                                                      H.g, H.c, H.af, H.r, H.e[0], omega);
+}
+
+// the last pre-sweep (e[cur] to e[nxt]) and the restriction in one pass
+template <int CK>
+__global__ __launch_bounds__(kTwoThreads) void kb_pre_restrict(const BSeg *segs,
+                                                               const uint16_t *bmap,
+                                                               const BFine *fine,
+                                                               const BLev<float> *lev,
+                                                               const BLev<float> *levH, int cur,
+                                                               int nxt, float omega) {
+  PSB_BSEG_BEGIN
+  const BLev<float> &L = lev[sg_.sys];
+  if (F.st->done || sp.bl >= L.two.nblocks) return;
+  const BLev<float> &H = levH[sg_.sys];
+  pre_restrict_body<float, 4, float, true, CK>(sp.bl, L.g, L.matflux(), L.r, L.e[cur], L.e[nxt],
+                                               L.af, H.g, H.c, H.af, H.r, H.e[0], omega, omega,
+                                               L.two);
+}
+
+// both post-sweeps in one pass (the prolongation as in kb_jacobi)
+template <int CK, bool RHO>
+__global__ __launch_bounds__(kTwoThreads) void kb_post_two(const BSeg *segs, const uint16_t *bmap,
+                                                           const BFine *fine,
+                                                           const BLev<float> *lev,
+                                                           const BLev<float> *levH, int cur,
+                                                           int nxt, int outH, float cfac,
+                                                           float omega, Work w, bool flex) {
+  PSB_BSEG_BEGIN
+  if (F.st->done) return;
+  const BLev<float> &L = lev[sg_.sys];
+  const BLev<float> &H = levH[sg_.sys];
+  TwoProl<float, 4, CK> pr{L.e[cur], H.kcyc ? H.kz : H.e[outH], L.af, H.kcyc ? 1.0f : cfac,
+                           L.g.sI, H.g.sI, H.sI, H.sJ, H.g.nz};
+  post_two_body<float, 4, float, true, CK, RHO>(sp.bl, L.g, L.matflux(), L.r, pr, L.e[nxt], omega,
+                                                1.0f, L.af, RHO && flex ? F.q : nullptr, w,
+                                                L.two);
 }
 
 // K-cycle steps on level `lev` of the systems of the list (kc_av_body and

@@ -164,9 +164,9 @@ struct TwoAt {
   uint32_t P, HP, Pn, Pt;  // cells in a plane: own and halo vector, j + 1, k + V
 };
 template <int V>
-__device__ __forceinline__ TwoAt two_at(const Grid &g, const TwoShape &s) {
+__device__ __forceinline__ TwoAt two_at(const Grid &g, const TwoShape &s, int wi) {
   TwoAt a;
-  const int wi = xcd_block(), per = s.ntj * s.ntk;
+  const int per = s.ntj * s.ntk;
   const int slab = wi / per, tile = wi - slab * per;
   const int tj = tile / s.ntk, tk = tile - tj * s.ntk;
   const int nv = g.nz / V, t = (int)threadIdx.x;
@@ -372,14 +372,15 @@ __device__ __forceinline__ void two_march(const Grid &g, const DMat<M> &A, const
 // r - A eout with the coarse level's first sweep (as k_jacobi and k_restrict,
 // CI = CJ = 2).  A coarse cell's sum runs in (i, j, k) order: the even row's
 // thread adds its own residuals and, a step later, the odd row's from LDS.
+// (block wi of s.nblocks)
 template <typename T, int V, typename M, bool FLUX, int CK>
-__global__ __launch_bounds__(kTwoThreads) void k_pre_restrict(
-    Grid g, DMat<M> A, const T *r, const T *e, T *eout, const uint8_t *af, Grid gH, const T *cH,
-    const uint8_t *afH, T *rH, T *eH1, T omega, T omegaH, const DevState *st, TwoShape s) {
-  if (skip_done(st, g.N)) return;
+__device__ __forceinline__ void pre_restrict_body(int wi, Grid g, DMat<M> A, const T *r,
+                                                  const T *e, T *eout, const uint8_t *af, Grid gH,
+                                                  const T *cH, const uint8_t *afH, T *rH, T *eH1,
+                                                  T omega, T omegaH, TwoShape s) {
   extern __shared__ __align__(16) char two_lds[];
   T *const lds = reinterpret_cast<T *>(two_lds);
-  const TwoAt a = two_at<V>(g, s);
+  const TwoAt a = two_at<V>(g, s, wi);
   const int pitch = s.KT * V, nt = (s.RT - 2) / 2 * pitch;
   T *const lt = lds + (2 * (s.RT + 2) + 2 * s.RT) * pitch;  // odd rows' residuals, two planes
   const bool odd = (a.rr & 1) == 0;  // output row rr - 1
@@ -469,20 +470,32 @@ __global__ __launch_bounds__(kTwoThreads) void k_pre_restrict(
   store();
 }
 
+template <typename T, int V, typename M, bool FLUX, int CK>
+__global__ __launch_bounds__(kTwoThreads) void k_pre_restrict(
+    Grid g, DMat<M> A, const T *r, const T *e, T *eout, const uint8_t *af, Grid gH, const T *cH,
+    const uint8_t *afH, T *rH, T *eH1, T omega, T omegaH, const DevState *st, TwoShape s) {
+  if (skip_done(st, g.N)) return;
+  pre_restrict_body<T, V, M, FLUX, CK>(xcd_block(), g, A, r, e, eout, af, gH, cH, afH, rH, eH1,
+                                       omega, omegaH, s);
+}
+
 // the two post-sweeps of a level, the prolongation of eH fused into the first
 // (as k_jacobi with PROL, then without); RHO: the finest level, whose second
 // sweep leaves z times zscale and the rho partials (rho_accq), one set per
-// block
+// block (zeros past the last)
 template <typename T, int V, typename M, bool FLUX, int CK, bool RHO>
-__global__ __launch_bounds__(kTwoThreads) void k_post_two(Grid g, DMat<M> A, const T *r,
-                                                          TwoProl<T, V, CK> pr, T *eout, T omega,
-                                                          T zscale, const uint8_t *af,
-                                                          const T *qf, const DevState *st, Work w,
-                                                          TwoShape s) {
-  if (skip_done(st, g.N)) return;
+__device__ __forceinline__ void post_two_body(int wi, Grid g, DMat<M> A, const T *r,
+                                              TwoProl<T, V, CK> pr, T *eout, T omega, T zscale,
+                                              const uint8_t *af, const T *qf, Work w,
+                                              TwoShape s) {
+  if (wi >= s.nblocks) {
+    if (RHO && threadIdx.x < kRhoParts)
+      w.partial[(size_t)blockIdx.x * kRhoParts + threadIdx.x] = 0.0;
+    return;
+  }
   extern __shared__ __align__(16) char two_lds[];
   T *const lds = reinterpret_cast<T *>(two_lds);
-  const TwoAt a = two_at<V>(g, s);
+  const TwoAt a = two_at<V>(g, s, wi);
   const uint32_t oT = a.P * (uint32_t)sizeof(T);
   double acc[kRhoParts] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   int count = 0;   // active cells (an integer takes half the registers)
@@ -538,6 +551,17 @@ __global__ __launch_bounds__(kTwoThreads) void k_post_two(Grid g, DMat<M> A, con
       w.partial[(size_t)blockIdx.x * kRhoParts + threadIdx.x] = t;
     }
   }
+}
+
+template <typename T, int V, typename M, bool FLUX, int CK, bool RHO>
+__global__ __launch_bounds__(kTwoThreads) void k_post_two(Grid g, DMat<M> A, const T *r,
+                                                          TwoProl<T, V, CK> pr, T *eout, T omega,
+                                                          T zscale, const uint8_t *af,
+                                                          const T *qf, const DevState *st, Work w,
+                                                          TwoShape s) {
+  if (skip_done(st, g.N)) return;
+  post_two_body<T, V, M, FLUX, CK, RHO>(xcd_block(), g, A, r, pr, eout, omega, zscale, af, qf, w,
+                                        s);
 }
 
 }  // namespace psb
