@@ -3097,8 +3097,13 @@ int psb_project_device(psb_ctx *C, const double *d_rho, const double *d_p, doubl
   if (!C->have_matrix || !C->metrics.dxc) return PSB_ENOTREADY;
   return guarded(C, [&]() {
     const Grid &g = C->g;
-    hipLaunchKernelGGL(k_project, dim3(grid_blocks(g.N)), dim3(kBlock), 0, C->stream, g,
-                       C->metrics, d_rho, C->off_dev, d_p, dt, mask, d_u, d_v, d_w);
+    // slabs of up to 16 planes, fewer where that leaves the chip idle
+    const int ntiles = (g.ny * g.nz + kBlock - 1) / kBlock;
+    int TI = 16;
+    while (TI > 1 && (long long)ntiles * ((g.nx + TI - 1) / TI) < 2048) TI /= 2;
+    hipLaunchKernelGGL(k_project, dim3(ntiles * ((g.nx + TI - 1) / TI)), dim3(kBlock), 0,
+                       C->stream, g, C->metrics, d_rho, C->off_dev, d_p, dt, mask, d_u, d_v, d_w,
+                       TI, ntiles);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(C->stream));
     return (int)PSB_OK;

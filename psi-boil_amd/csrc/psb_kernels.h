@@ -2003,50 +2003,82 @@ static __global__ void k_rhs_center(Grid g, double *b, const uint8_t *off, const
     if (!(off && off[P])) b[P] = b[P] - mean;
 }
 
-// Momentum::project (momentum_project.cpp:10-76), one cell per thread: the
-// cell's west, south and bottom faces when they are interior faces (the wall
-// faces stay, staggered_set_indices.cpp:9-19) take
-// (p_nb - p_P) / rho_f * dt / d with rho_f = (rho_P + rho_nb) / 2
-// (property_value.cpp:18-32) and d the centre distance (dxw, dys, dzb).
-// With solid cells (off) the body form: faces between two fluid cells only,
-// rounded as (p_nb - p_P) * dt / rho_f / d (:50-70).  mask bits 0/1/2 select
-// u, v, w (Momentum's ifull / jfull / kfull).  64 B per cell: p, rho, and
-// the three face arrays read and written.
+// Momentum::project (momentum_project.cpp:10-76): a cell's west, south and
+// bottom faces when they are interior faces (the wall faces stay,
+// staggered_set_indices.cpp:9-19) take (p_nb - p_P) / rho_f * dt / d with
+// rho_f = (rho_P + rho_nb) / 2 (property_value.cpp:18-32) and d the centre
+// distance (dxw, dys, dzb).  With solid cells (off) the body form: faces
+// between two fluid cells only, rounded as (p_nb - p_P) * dt / rho_f / d
+// (:50-70).  mask bits 0/1/2 select u, v, w (Momentum's ifull / jfull / kfull).
+// 64 B per cell: p, rho, and the three face arrays read and written.
+// A thread walks planes [slab * TI, + TI) at one (j, k): the plane's index is
+// found once, p and rho of the plane below stay in registers, and the next
+// plane's loads are under way while this one's six divisions are computed
+// (201 x 180 x 222: 110 us, 4.7 TB/s, against 130 for one cell at a time; with
+// 8 planes a slab 110, with 32 115 and with 64 133, when blocks are few).
 static __global__ __launch_bounds__(kBlock) void k_project(Grid g, DevMetrics m,
                                                            const double *rho, const uint8_t *off,
                                                            const double *p, double dt, int mask,
-                                                           double *u, double *v, double *wv) {
-  const int gy = g.ny + 2, gz = g.nz + 2;
-  const size_t ny = g.ny, nz = g.nz;
-  for (int P = blockIdx.x * blockDim.x + threadIdx.x; P < g.N; P += gridDim.x * blockDim.x) {
-    int i, j, k;
-    g.ijk(P, i, j, k);
-    auto R = [&](int a, int b, int c) {
-      return rho[((size_t)(a + 1) * gy + (b + 1)) * gz + (c + 1)];
-    };
-    const double pp = p[P], rp = R(i, j, k);
-    const bool fluid = !(off && off[P]);
-    if ((mask & 1) && i > 0) {
-      const int Q = P - g.sI;
-      const double rf = 0.5 * (rp + R(i - 1, j, k));
-      double &f = u[P];  // face i of (nx+1) x ny x nz: same index as the cell
-      if (!off) f += (p[Q] - pp) / rf * dt / m.dxw[i];
-      else if (fluid && !off[Q]) f += (p[Q] - pp) * dt / rf / m.dxw[i];
+                                                           double *u, double *v, double *wv,
+                                                           int TI, int ntiles) {
+  const int slab = (int)blockIdx.x / ntiles, tile = (int)blockIdx.x - slab * ntiles;
+  const int t = tile * kBlock + (int)threadIdx.x, plane = g.ny * g.nz;
+  if (t >= plane) return;
+  const int j = t / g.nz, k = t - j * g.nz;
+  const int i0 = slab * TI, i1 = min(i0 + TI, g.nx);
+  const size_t gz = g.nz + 2, gp = (size_t)(g.ny + 2) * gz;
+  const double *R = rho + gp + (size_t)(j + 1) * gz + k + 1;  // cell (0, j, k)
+  const bool fu = mask & 1, fv = (mask & 2) && j > 0, fw = (mask & 4) && k > 0;
+  double *const U = fu ? u + t : nullptr;
+  double *const Vf = fv ? v + (size_t)j * g.nz + k : nullptr;
+  double *const Wf = fw ? wv + (size_t)j * (g.nz + 1) + k : nullptr;
+  const size_t pv = (size_t)(g.ny + 1) * g.nz, pw = (size_t)g.ny * (g.nz + 1);
+  const int tS = j > 0 ? t - g.nz : t, tB = k > 0 ? t - 1 : t;
+  const size_t rS = j > 0 ? gz : 0, rB = k > 0 ? 1 : 0;
+  struct Cell {
+    double p, pS, pB, r, rS, rB, u, v, w;
+  };
+  auto load = [&](int i) {
+    Cell c;
+    const double *P = p + (size_t)i * plane, *Q = R + (size_t)i * gp;
+    c.p = P[t];
+    c.pS = P[tS];
+    c.pB = P[tB];
+    c.r = *Q;
+    c.rS = *(Q - rS);
+    c.rB = *(Q - rB);
+    c.u = fu ? U[(size_t)i * plane] : 0.0;
+    c.v = fv ? Vf[i * pv] : 0.0;
+    c.w = fw ? Wf[i * pw] : 0.0;
+    return c;
+  };
+  const double dS = m.dys[j], dB = m.dzb[k];
+  const int ib = max(i0 - 1, 0);
+  double pW = p[(size_t)ib * plane + t], rW = R[(size_t)ib * gp];
+  Cell c = load(i0);
+  for (int i = i0; i < i1; i++) {
+    const Cell n = load(min(i + 1, i1 - 1));
+    const uint8_t *o = off ? off + (size_t)i * plane : nullptr;
+    const bool fluid = !(o && o[t]);
+    if (fu && i > 0) {
+      const double rf = 0.5 * (c.r + rW);
+      if (!off) U[(size_t)i * plane] = c.u + (pW - c.p) / rf * dt / m.dxw[i];
+      else if (fluid && !(o - plane)[t])
+        U[(size_t)i * plane] = c.u + (pW - c.p) * dt / rf / m.dxw[i];
     }
-    if ((mask & 2) && j > 0) {
-      const int Q = P - g.nz;
-      const double rf = 0.5 * (rp + R(i, j - 1, k));
-      double &f = v[((size_t)i * (ny + 1) + j) * nz + k];
-      if (!off) f += (p[Q] - pp) / rf * dt / m.dys[j];
-      else if (fluid && !off[Q]) f += (p[Q] - pp) * dt / rf / m.dys[j];
+    if (fv) {
+      const double rf = 0.5 * (c.r + c.rS);
+      if (!off) Vf[i * pv] = c.v + (c.pS - c.p) / rf * dt / dS;
+      else if (fluid && !o[tS]) Vf[i * pv] = c.v + (c.pS - c.p) * dt / rf / dS;
     }
-    if ((mask & 4) && k > 0) {
-      const int Q = P - 1;
-      const double rf = 0.5 * (rp + R(i, j, k - 1));
-      double &f = wv[((size_t)i * ny + j) * (nz + 1) + k];
-      if (!off) f += (p[Q] - pp) / rf * dt / m.dzb[k];
-      else if (fluid && !off[Q]) f += (p[Q] - pp) * dt / rf / m.dzb[k];
+    if (fw) {
+      const double rf = 0.5 * (c.r + c.rB);
+      if (!off) Wf[i * pw] = c.w + (c.pB - c.p) / rf * dt / dB;
+      else if (fluid && !o[tB]) Wf[i * pw] = c.w + (c.pB - c.p) * dt / rf / dB;
     }
+    pW = c.p;
+    rW = c.r;
+    c = n;
   }
 }
 
