@@ -215,12 +215,16 @@ void cg_xr(psb_ctx *C, const Grid &g, const T *c, const T *p, const T *q, T *x, 
   const Metric m = mt ? *mt : metric(C);
   const Fold f{npq, pq_work(C).partial, nullptr};
   {
-    // x, r, p, q, c in; x, r (and e1) out
-    ProbeScope ps(C, PSB_K_CG_XR, g, (DIAG ? 7 : 8) * sizeof(T));
+    // x, r, p, q (and c) in; x, r (and e1) out
+    ProbeScope ps(C, PSB_K_CG_XR, g, (DIAG ? 7 : e1 ? 8 : 6) * sizeof(T));
     with_v<T>(g, [&](auto vt) {
       constexpr int V = decltype(vt)::value;
-      hipLaunchKernelGGL((k_cg_xr<T, V, DIAG>), dim3(nblocks<T>(g)), dim3(kBlock), 0, C->stream,
-                         g, c, m, p, q, x, r, e1, omega, st, C->work, f);
+      if (DIAG || e1)
+        hipLaunchKernelGGL((k_cg_xr<T, V, DIAG>), dim3(nblocks<T>(g)), dim3(kBlock), 0,
+                           C->stream, g, c, m, p, q, x, r, e1, omega, st, C->work, f);
+      else
+        hipLaunchKernelGGL((k_cg_xr<T, V, false, false>), dim3(nblocks<T>(g)), dim3(kBlock), 0,
+                           C->stream, g, c, m, p, q, x, r, e1, omega, st, C->work, f);
     });
   }
   finalize<3>(C, op >= 0 ? op : DIAG ? FIN_XR_DIAG : FIN_XR_AC, nblocks<T>(g), st);
@@ -489,8 +493,7 @@ bool two_shape(const psb_ctx *C, const Grid &g, TwoShape &s) {
     for (int R = 2; (R + 2) * KT <= kTwoThreads; R += 2) {
       const size_t lds = (size_t)(2 * (R + 4) + 2 * (R + 2) + R) * KT * V;
       if (lds * sizeof(T) > 150 * 1024) break;
-      // (blocks share a compute unit where their waves spread evenly over its SIMDs)
-      const int waves = ((R + 2) * KT + 63) / 64, per_cu = waves > 4 ? 1 : 12 / (waves > 2 ? 4 : 2);
+      const int waves = ((R + 2) * KT + 63) / 64, per_cu = std::max(1, 12 / waves);
       const long long nt = (long long)((g.ny + R - 1) / R) * ntk;
       for (int TI = 2; TI < g.nx + 2; TI += 2) {
         const long long nb = nt * ((g.nx + TI - 1) / TI);
@@ -514,19 +517,26 @@ bool two_shape(const psb_ctx *C, const Grid &g, TwoShape &s) {
   return best > 0.0;
 }
 
-// the last pre-sweep of level lv (e to eout) and the restriction to cL in one
-// pass; false where the level does not suit it
+// the last pre-sweep of level lv (e to eout; e NULL: from the first sweep omega
+// r / c, formed in the pass) and the restriction to cL in one pass; false where
+// the level does not suit it
 template <typename T, typename M, bool FLUX>
 void pre_restrict_m(psb_ctx *C, const Level<T> &lv, DMat<M> A, const T *e, T *eout, Level<T> &cL,
                     T omega, T omegaH, DevState *st, const TwoShape &s) {
   constexpr int V = vmax<T>();
-  auto go = [&](auto ck) {
-    hipLaunchKernelGGL((k_pre_restrict<T, V, M, FLUX, decltype(ck)::value>), dim3(s.nblocks),
-                       dim3(s.threads), s.lds * sizeof(T), C->stream, lv.g, A, lv.r, e, eout,
-                       lv.aflag, cL.g, cL.c, cL.aflag, cL.r, cL.e[0], omega, omegaH, st, s);
+  auto go = [&](auto ck, auto first) {
+    hipLaunchKernelGGL(
+        (k_pre_restrict<T, V, M, FLUX, decltype(ck)::value, decltype(first)::value>),
+        dim3(s.nblocks), dim3(s.threads), s.lds * sizeof(T), C->stream, lv.g, A, lv.r, e, lv.c,
+        T(omega / lv.scale), eout, lv.aflag, cL.g, cL.c, cL.aflag, cL.r, cL.e[0], omega, omegaH,
+        st, s);
   };
-  if (cL.CK == 2) go(std::integral_constant<int, 2>());
-  else go(std::integral_constant<int, 1>());
+  auto with_ck = [&](auto first) {
+    if (cL.CK == 2) go(std::integral_constant<int, 2>(), first);
+    else go(std::integral_constant<int, 1>(), first);
+  };
+  if (e) with_ck(std::false_type());
+  else with_ck(std::true_type());
 }
 template <typename T>
 bool pre_restrict(psb_ctx *C, const Level<T> &lv, const T *e, T *eout, Level<T> &cL, T omega,
@@ -547,6 +557,25 @@ bool pre_restrict(psb_ctx *C, const Level<T> &lv, const T *e, T *eout, Level<T> 
     pre_restrict_m<T, T, false>(C, lv, lv.mat(), e, eout, cL, omega, omegaH, st, s);
   }
   return true;
+}
+
+template <typename T>
+bool tail_at(const psb_ctx *C, const Hier<T> &H, int l);
+
+// whether the finest level's first sweep is formed in pre_restrict's pass, so that
+// the CG's x/r step need neither write it nor read c (6 arrays instead of 8; the
+// pass reads c in e's place and divides).  Measured, us, x/r step + pass: 512^3
+// FP32 836 + 612 -> 626 + 719, 256^3 FP32 112 + 87 -> 83 + 98 and FP64 219 + 217
+// -> 168 + 210, 128^3 FP32, which does not leave the caches, 12.7 + 17.4 -> 10.2 +
+// 20.3: the line lies between.
+constexpr int kFirstCells = 1 << 22;
+template <typename T>
+bool first_in_pass(const psb_ctx *C, const Hier<T> &H, int nu1) {
+  const Level<T> &lv = H.L[0], &cL = H.L[1];
+  TwoShape s{};
+  return nu1 == 2 && lv.g.N >= kFirstCells && !lv.ae &&
+         !(std::is_same<T, float>::value && !lv.d) && !tail_at(C, H, 0) && cL.CI == 2 &&
+         cL.CJ == 2 && two_shape<T>(C, lv.g, s);
 }
 
 // the two post-sweeps of level lv in one pass (e and the correction eH of cL
@@ -1336,7 +1365,9 @@ T *vcycle(psb_ctx *C, Hier<T> &H, int l, DevState *st, int nu1, int nu2, T omega
   for (int s = 1 + done; s < nu1; s++) {
     const int nxt = (cur + 1) % 3;
     if (s == nu1 - 1)
-      restricted = pre_restrict<T>(C, lv, lv.e[cur], lv.e[nxt], cL, omega, T(omega / cL.scale), st);
+      restricted = pre_restrict<T>(
+          C, lv, l == 0 && rho0 && first_in_pass(C, H, nu1) ? nullptr : lv.e[cur], lv.e[nxt], cL,
+          omega, T(omega / cL.scale), st);
     if (!restricted)
       jacobi<T, false>(C, lv, lv.e[cur], lv.e[nxt], nullptr, nullptr, T(0), omega, st);
     cur = nxt;
@@ -1412,7 +1443,8 @@ void ac_iteration(psb_ctx *C, Hier<T> &H, KrylovVecs<T> &K, DevState *st, int pa
     else
       npq = cg_pq<T, true, false>(C, f.g, f.mat(), z, pold, pnew, K.q, f.aflag, st);
   }
-  cg_xr<T, false>(C, f.g, f.c, pnew, K.q, K.x, K.r, f.e[0], T(omega / f.scale), st, npq, xr_op);
+  cg_xr<T, false>(C, f.g, f.c, pnew, K.q, K.x, K.r,
+                  first_in_pass(C, H, nu1) ? nullptr : f.e[0], T(omega / f.scale), st, npq, xr_op);
 }
 
 void destroy_graph(Graph &gr) {

@@ -120,7 +120,8 @@ __global__ __launch_bounds__(kTwoThreads) void kb_pre_restrict(const BSeg *segs,
   const BLev<float> &L = lev[sg_.sys];
   if (F.st->done || sp.bl >= L.two.nblocks) return;
   const BLev<float> &H = levH[sg_.sys];
-  pre_restrict_body<float, 4, float, true, CK>(sp.bl, L.g, L.matflux(), L.r, L.e[cur], L.e[nxt],
+  pre_restrict_body<float, 4, float, true, CK>(sp.bl, L.g, L.matflux(), L.r,
+                                               TwoArr<float, 4>{L.e[cur], L.g.sI}, L.e[nxt],
                                                L.af, H.g, H.c, H.af, H.r, H.e[0], omega, omega,
                                                L.two);
 }

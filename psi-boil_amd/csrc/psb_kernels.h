@@ -644,17 +644,18 @@ __global__ __launch_bounds__(kBlock) void k_cg_pq(Grid g, DMat<T> A, const T *r_
     if (DIAG) {                                               \
       T z = R.v[u] * (T(1) / C.v[u]);                         \
       acc[2] += (double)(R.v[u] * z);                         \
-    } else {                                                  \
+    } else if (E1) {                                          \
       E.v[u] = omega * R.v[u] / C.v[u];                       \
     }                                                         \
   }                                                           \
   stv<T, V>(x + P, X);                                        \
   stv<T, V>(r + P, R);                                        \
-  if (!DIAG) stv<T, V>(e1 + P, E);
+  if (!DIAG && E1) stv<T, V>(e1 + P, E);
 
 // (get_alpha gives alpha, or false where the solve has stopped; in FP64 it is
 // called once the first loads are under way)
-template <typename T, int V, bool DIAG, class GetAlpha>
+// (E1 false: the V-cycle forms its first sweep itself; 6 arrays instead of 8)
+template <typename T, int V, bool DIAG, bool E1 = true, class GetAlpha>
 __device__ __forceinline__ void cg_xr_body(Span sp, const Grid &g, const T *c, const Metric &m,
                                            const T *p, const T *q, T *x, T *r, T *e1, T omega,
                                            const DevState *st, Work w, GetAlpha get_alpha) {
@@ -672,7 +673,8 @@ __device__ __forceinline__ void cg_xr_body(Span sp, const Grid &g, const T *c, c
     int qq = q0 + (int)threadIdx.x;
     const int Pf = (qq < q1 ? qq : 0) * V;
     VecN<T, V> Xn = ldv<T, V>(x + Pf), Rn = ldv<T, V>(r + Pf), Pn = ldv<T, V>(p + Pf),
-               Qn = ldv<T, V>(q + Pf), Cn = ldv<T, V>(c + Pf);
+               Qn = ldv<T, V>(q + Pf), Cn{};
+    if (E1) Cn = ldv<T, V>(c + Pf);
     double al;
     if (!get_alpha(al)) return;
     const T alpha = (T)al;
@@ -686,7 +688,7 @@ __device__ __forceinline__ void cg_xr_body(Span sp, const Grid &g, const T *c, c
       Rn = ldv<T, V>(r + Pnx);
       Pn = ldv<T, V>(p + Pnx);
       Qn = ldv<T, V>(q + Pnx);
-      Cn = ldv<T, V>(c + Pnx);
+      if (E1) Cn = ldv<T, V>(c + Pnx);
       PSB_CG_XR_CELL
     }
   } else {
@@ -695,7 +697,8 @@ __device__ __forceinline__ void cg_xr_body(Span sp, const Grid &g, const T *c, c
     const T alpha = (T)al;
     PSB_SPAN_BEGIN(g, V, sp)
     VecN<T, V> X = ldv<T, V>(x + P), R = ldv<T, V>(r + P), Pp = ldv<T, V>(p + P),
-               Q = ldv<T, V>(q + P), C = ldv<T, V>(c + P), E;
+               Q = ldv<T, V>(q + P), C{}, E;
+    if (E1) C = ldv<T, V>(c + P);
     PSB_CG_XR_CELL
     PSB_TILE_END
   }
@@ -703,11 +706,11 @@ __device__ __forceinline__ void cg_xr_body(Span sp, const Grid &g, const T *c, c
 }
 #undef PSB_CG_XR_CELL
 
-template <typename T, int V, bool DIAG>
+template <typename T, int V, bool DIAG, bool E1 = true>
 __global__ __launch_bounds__(kBlock) void k_cg_xr(Grid g, const T *c, Metric m, const T *p,
                                                   const T *q, T *x, T *r, T *e1, T omega,
                                                   DevState *st, Work w, Fold f) {
-  cg_xr_body<T, V, DIAG>(grid_span(), g, c, m, p, q, x, r, e1, omega, st, w, [&](double &al) {
+  cg_xr_body<T, V, DIAG, E1>(grid_span(), g, c, m, p, q, x, r, e1, omega, st, w, [&](double &al) {
     const int done = st->done;
     const double rho = st->rho;
     al = f.nprev > 0 ? fold_pq(f, st, rho) : st->alpha;

@@ -221,6 +221,32 @@ struct TwoArr {
   }
   __device__ __forceinline__ VecN<T, V> form(const Raw &x) const { return x; }
 };
+// the first sweep from zero, omega r / c, formed where it is used: the finest
+// level's operand needs neither its writing by the CG step before nor its c there
+template <typename T, int V>
+struct TwoFirst {
+  const T *r, *c;
+  T omega;
+  int sI;
+  struct At {
+    uint32_t o;
+  };
+  struct Raw {
+    VecN<T, V> R, C;
+  };
+  __device__ __forceinline__ At place(int j, int k, int nz) const {
+    return At{(uint32_t)(j * nz + k) * (uint32_t)sizeof(T)};
+  }
+  __device__ __forceinline__ Raw load(int i, const At &a) const {
+    return Raw{ldo<T, V>(r + (size_t)i * sI, a.o), ldo<T, V>(c + (size_t)i * sI, a.o)};
+  }
+  __device__ __forceinline__ VecN<T, V> form(const Raw &x) const {
+    VecN<T, V> o;
+#pragma unroll
+    for (int u = 0; u < V; u++) o.v[u] = omega * x.R.v[u] / x.C.v[u];
+    return o;
+  }
+};
 template <typename T, int V, int CK>
 struct TwoProl {
   const T *e, *eH;
@@ -373,11 +399,11 @@ __device__ __forceinline__ void two_march(const Grid &g, const DMat<M> &A, const
 // CI = CJ = 2).  A coarse cell's sum runs in (i, j, k) order: the even row's
 // thread adds its own residuals and, a step later, the odd row's from LDS.
 // (block wi of s.nblocks)
-template <typename T, int V, typename M, bool FLUX, int CK>
-__device__ __forceinline__ void pre_restrict_body(int wi, Grid g, DMat<M> A, const T *r,
-                                                  const T *e, T *eout, const uint8_t *af, Grid gH,
-                                                  const T *cH, const uint8_t *afH, T *rH, T *eH1,
-                                                  T omega, T omegaH, TwoShape s) {
+template <typename T, int V, typename M, bool FLUX, int CK, class B>
+__device__ __forceinline__ void pre_restrict_body(int wi, Grid g, DMat<M> A, const T *r, const B &e,
+                                                  T *eout, const uint8_t *af, Grid gH, const T *cH,
+                                                  const uint8_t *afH, T *rH, T *eH1, T omega,
+                                                  T omegaH, TwoShape s) {
   extern __shared__ __align__(16) char two_lds[];
   T *const lds = reinterpret_cast<T *>(two_lds);
   const TwoAt a = two_at<V>(g, s, wi);
@@ -430,7 +456,7 @@ __device__ __forceinline__ void pre_restrict_body(int wi, Grid g, DMat<M> A, con
     if (afH) act = ldflags<NC>(afH + p, QH);
   };
   two_march<T, V, M, FLUX>(
-      g, A, r, TwoArr<T, V>{e, g.sI}, omega, s, a, lds,
+      g, A, r, e, omega, s, a, lds,
       [&](int i) {
         if (a.out)
           sto<T, V>(eout + (size_t)i * g.sI, a.P * (uint32_t)sizeof(T),
@@ -470,13 +496,19 @@ __device__ __forceinline__ void pre_restrict_body(int wi, Grid g, DMat<M> A, con
   store();
 }
 
-template <typename T, int V, typename M, bool FLUX, int CK>
+// (FIRST: the operand is the first sweep om0 r / c, e is not read)
+template <typename T, int V, typename M, bool FLUX, int CK, bool FIRST>
 __global__ __launch_bounds__(kTwoThreads) void k_pre_restrict(
-    Grid g, DMat<M> A, const T *r, const T *e, T *eout, const uint8_t *af, Grid gH, const T *cH,
-    const uint8_t *afH, T *rH, T *eH1, T omega, T omegaH, const DevState *st, TwoShape s) {
+    Grid g, DMat<M> A, const T *r, const T *e, const T *c, T om0, T *eout, const uint8_t *af,
+    Grid gH, const T *cH, const uint8_t *afH, T *rH, T *eH1, T omega, T omegaH,
+    const DevState *st, TwoShape s) {
   if (skip_done(st, g.N)) return;
-  pre_restrict_body<T, V, M, FLUX, CK>(xcd_block(), g, A, r, e, eout, af, gH, cH, afH, rH, eH1,
-                                       omega, omegaH, s);
+  if constexpr (FIRST)
+    pre_restrict_body<T, V, M, FLUX, CK>(xcd_block(), g, A, r, TwoFirst<T, V>{r, c, om0, g.sI},
+                                         eout, af, gH, cH, afH, rH, eH1, omega, omegaH, s);
+  else
+    pre_restrict_body<T, V, M, FLUX, CK>(xcd_block(), g, A, r, TwoArr<T, V>{e, g.sI}, eout, af,
+                                         gH, cH, afH, rH, eH1, omega, omegaH, s);
 }
 
 // the two post-sweeps of a level, the prolongation of eH fused into the first
