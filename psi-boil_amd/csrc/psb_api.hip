@@ -231,17 +231,24 @@ void cg_xr(psb_ctx *C, const Grid &g, const T *c, const T *p, const T *q, T *x, 
 }
 
 // A run of `n` CG iterations with the diagonal preconditioner (cg.cpp:66-160),
-// FP64.  On grids up to kFoldCells both scalar steps are folded into the
+// FP64.  On small grids (cg_di_fold) both scalar steps are folded into the
 // streaming kernels (k_cg_pq_di, k_cg_xr_di): two launches an iteration instead
 // of four, the state handed from st to st2 and back; the last iteration's step
-// ends in st (unless `last` is false: nobody asks for it).  Measured: 64^3 6.3
-// -> 4.5 ms per 334 iterations (5.9 + 4.7 us of kernels and two nodes), 57x45x39
-// 12.7 -> 8.8 ms, two V-cycles of 96^3 12.5 -> 8.3 ms (folding up to 2^19 cells
-// only: 8.9).  The line: every block reads every partial, which at 96^3 (1728
-// blocks) brings the pair from 25 to 32 us, as much as the two launches cost; on
-// larger grids, whose kernels stream from HBM, only alpha is folded (fold_pq).
+// ends in st (unless `last` is false: nobody asks for it).  On larger grids only
+// alpha is folded (fold_pq).
+// The line: every block reads every partial, which grows with the blocks squared
+// and at some thousand of them costs what the two launches cost.  us an
+// iteration, folded / not, two-wide cells: 64^3 11.3 / 13.3, 80^3 20.3 / 21.6,
+// 96 x 72 x 72 21.5 / 22.0, 88 x 84 x 84 26.3 / 26.0, 96^3 30.6 / 29.3, 156 x 41 x
+// 146 31.7 / 30.7; scalar cells (odd nz): 57 x 45 x 39 10.9 / 13.1, 50 x 50 x 59
+// 15.9 / 14.8, 80 x 80 x 79 36.2 / 25.8.  The reference's cycle runs its levels'
+// solves for a fixed number of iterations, most of them after they have stopped,
+// where only the launches count: two cycles of 96^3 8.3 ms folded up to 2^20
+// two-wide cells, 8.9 up to 2^19 (12.5 not folded).
 constexpr int kFoldCells = 1 << 20;
-bool cg_di_fold(const psb_ctx *C, const Grid &g) { return C->fold && g.N <= kFoldCells; }
+bool cg_di_fold(const psb_ctx *C, const Grid &g, bool cycle = false) {
+  return C->fold && g.N <= (!vec_ok<double>(g) ? 1 << 17 : cycle ? kFoldCells : 1 << 19);
+}
 // q: two arrays with the fold (z of the iteration before is read from one,
 // q[0] at the start, while A p goes to the other); n even unless it ends there
 template <bool SYM>
@@ -249,7 +256,7 @@ void cg_di_run(psb_ctx *C, const Grid &g, DMat<double> A, double *r, double *con
                double *const q[2], double *x, DevState *st, DevState *st2, int n,
                const Metric *mt = nullptr, bool last = true) {
   const int nxr = nblocks<double>(g);
-  const bool fold = cg_di_fold(C, g);
+  const bool fold = cg_di_fold(C, g, mt != nullptr);
   DevState *cur = st;
   for (int it = 0; it < n; it++) {
     const double *pold = p[it & 1];
@@ -1801,11 +1808,14 @@ void solve_bicgs_diag(psb_ctx *C, double *x, const double *b, const psb_stop *p,
   read_state(C, C->st64);
   const int chunk = chunk_of(p);
   const int nb = nblocks<double>(g);
-  // on grids up to kFoldCells the scalar steps are folded into the kernels that
+  // on small grids the scalar steps are folded into the kernels that
   // use them (as cg_di_run): three launches an iteration instead of six.
   // Measured, 65x48x80, 40 iterations: 1.26 -> 0.94 ms (7.3 + 7.1 + 4.7 us of
-  // kernels and 9.3 of steps became 7.8 + 6.5 + 5.3)
-  const bool fold = cg_di_fold(C, g);
+  // kernels and 9.3 of steps became 7.8 + 6.5 + 5.3).  The line (see cg_di_fold),
+  // us an iteration, folded / not: two-wide cells 80^3 31.2 / 35.4, 92 x 90 x 90
+  // 45.4 / 47.7, 96^3 50.5 / 51.4, 156 x 41 x 146 54.8 / 53.6; scalar cells 70 x 66
+  // x 67 32.4 / 35.4, 76 x 70 x 71 38.2 / 38.5, 80 x 80 x 79 46.3 / 44.9
+  const bool fold = C->fold && nb <= 1536;
   Work w1 = pq_work(C), w2 = C->work, w3{C->work.partial + (size_t)kMaxBlocks * 3};
   if (!fold) w1 = w3 = w2;
   auto body = [&]() {
@@ -2354,7 +2364,7 @@ void ref_cg(psb_ctx *C, int l, int maxit, double res_rat, double res_tol, double
   zero(C, p0, g.N);
   zero(C, p1, g.N);
   double *const p[2] = {p0, p1}, *const qz[2] = {q, H.K[l][4]};
-  start<double, SYM, 0>(C, g, lv.mat(), lv.r, lv.e[0], r, cg_di_fold(C, g) ? q : nullptr, 0.0, st,
+  start<double, SYM, 0>(C, g, lv.mat(), lv.r, lv.e[0], r, cg_di_fold(C, g, true) ? q : nullptr, 0.0, st,
                         &H.M[l]);
   cg_di_run<SYM>(C, g, lv.mat(), r, p, qz, lv.e[0], st, C->st64b, maxit, &H.M[l], verdict);
 }

@@ -2027,7 +2027,8 @@ static __global__ __launch_bounds__(kBlock) void k_project(Grid g, DevMetrics m,
   const int slab = (int)blockIdx.x / ntiles, tile = (int)blockIdx.x - slab * ntiles;
   const int t = tile * kBlock + (int)threadIdx.x, plane = g.ny * g.nz;
   if (t >= plane) return;
-  const int j = t / g.nz, k = t - j * g.nz;
+  int none, j, k;
+  g.ijk(t, none, j, k);
   const int i0 = slab * TI, i1 = min(i0 + TI, g.nx);
   const size_t gz = g.nz + 2, gp = (size_t)(g.ny + 2) * gz;
   const double *R = rho + gp + (size_t)(j + 1) * gz + k + 1;  // cell (0, j, k)
@@ -2060,7 +2061,8 @@ static __global__ __launch_bounds__(kBlock) void k_project(Grid g, DevMetrics m,
   double pW = p[(size_t)ib * plane + t], rW = R[(size_t)ib * gp];
   Cell c = load(i0);
   for (int i = i0; i < i1; i++) {
-    const Cell n = load(min(i + 1, i1 - 1));
+    Cell n = c;
+    if (i + 1 < i1) n = load(i + 1);
     const uint8_t *o = off ? off + (size_t)i * plane : nullptr;
     const bool fluid = !(o && o[t]);
     if (fu && i > 0) {
