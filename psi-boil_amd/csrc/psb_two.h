@@ -22,7 +22,7 @@
 //   first pair, FP16 copy: 256^3 87 / 78 + 67, 128^3 18 / 11.5 + 9.3, 32^3 7.1 / 4.5 + 5.5
 //   first pair, FP64:      256^3 216 / 399, 128^3 31 / 25 + 21, 32^3 6.7 / 3.9 + 4.9
 //   post-sweeps, FP16 copy: 256^3 100 / 76 + 81, 128^3 18.6 / 11.5 + 11.7, 32^3 8.2 / 4.5 + 4.7
-//   post-sweeps, FP64:      256^3 324 / 195 + 214, 128^3 25 / 25 + 21, 32^3 6.4 / 4.6 + 4.6
+//   post-sweeps, FP64:      256^3 278 / 195 + 214, 128^3 25 / 25 + 21, 32^3 6.4 / 4.6 + 4.6
 // The arithmetic is the separate kernels' (gather_c), so that the results are
 // bit-identical; only the rho partials are summed over other blocks.
 #pragma once
