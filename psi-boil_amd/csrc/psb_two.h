@@ -155,7 +155,7 @@ struct TwoRow {
 
 // a block's tile and slab, a thread's place in it
 struct TwoAt {
-  int rr, kk, j, k;     // tile row and vector, cell coordinates (clamped into the grid)
+  int rr, kk, j, k;     // tile row and vector, cell coordinates (clamped into tile and grid)
   int hk, hj, hrow;     // halo vector of the stage 1 operand this thread loads
   int i0, i1;           // the slab's output planes
   bool in, out, halo;   // takes part in stage 1 / stage 2, loads a halo vector
@@ -163,20 +163,27 @@ struct TwoAt {
   int os, on, ob, ot;   // neighbours in an LDS plane
   uint32_t P, HP, Pn, Pt;  // cells in a plane: own and halo vector, j + 1, k + V
 };
+// thread t of block wi.  A block has whole waves, so that its last threads can
+// lie past the tile: they write nothing, and their place is in the tile's last
+// row, so that what they read with the others (and use for nothing) is inside
+// the block's LDS.  (A branch around that read instead costs the FP64 post-sweeps
+// eight more spilled registers: 256^3 solve 29.8 against 29.5 ms.)
 template <int V>
-__device__ __forceinline__ TwoAt two_at(const Grid &g, const TwoShape &s, int wi) {
+__host__ __device__ __forceinline__ TwoAt two_place(const Grid &g, const TwoShape &s, int wi,
+                                                    int t) {
   TwoAt a;
   const int per = s.ntj * s.ntk;
   const int slab = wi / per, tile = wi - slab * per;
   const int tj = tile / s.ntk, tk = tile - tj * s.ntk;
-  const int nv = g.nz / V, t = (int)threadIdx.x;
+  const int nv = g.nz / V;
   const bool split = s.KO < s.KT;
-  a.rr = t / s.KT;
-  a.kk = t - a.rr * s.KT;
+  const int rr = t / s.KT;
+  a.rr = rr < s.RT ? rr : s.RT - 1;
+  a.kk = t - rr * s.KT;
   const int j0 = tj * (s.RT - 2) - 1, k0 = split ? tk * s.KO - 1 : 0;
-  const int j = j0 + a.rr, kv = k0 + a.kk;
+  const int j = j0 + rr, kv = k0 + a.kk;
   const bool kin = kv >= 0 && kv < nv;
-  a.in = a.rr < s.RT && j >= 0 && j < g.ny && kin;
+  a.in = rr < s.RT && j >= 0 && j < g.ny && kin;
   a.out = a.in && a.rr >= 1 && a.rr < s.RT - 1 && (!split || (a.kk >= 1 && a.kk <= s.KO));
   a.j = a.in ? j : 0;
   a.k = a.in ? kv * V : 0;
@@ -187,8 +194,8 @@ __device__ __forceinline__ TwoAt two_at(const Grid &g, const TwoShape &s, int wi
   a.hj = a.halo ? hj : 0;
   a.hk = a.halo ? hkv * V : 0;
   a.hrow = (t < s.KT ? 0 : s.RT + 1) * s.KT + hkk;
-  a.i0 = __builtin_amdgcn_readfirstlane(slab * s.TI);  // (the division left it in a VGPR)
-  a.i1 = min(a.i0 + s.TI, g.nx);
+  a.i0 = slab * s.TI;
+  a.i1 = a.i0 + s.TI < g.nx ? a.i0 + s.TI : g.nx;
   a.hn = a.j < g.ny - 1;
   a.ht = a.k + V < g.nz;
   a.os = a.j > 0 ? -s.KT * V : 0;
@@ -199,6 +206,13 @@ __device__ __forceinline__ TwoAt two_at(const Grid &g, const TwoShape &s, int wi
   a.HP = (uint32_t)(a.hj * g.nz + a.hk);
   a.Pn = a.hn ? a.P + g.nz : a.P;
   a.Pt = a.ht ? a.P + V : a.P;
+  return a;
+}
+template <int V>
+__device__ __forceinline__ TwoAt two_at(const Grid &g, const TwoShape &s, int wi) {
+  TwoAt a = two_place<V>(g, s, wi, (int)threadIdx.x);
+  a.i0 = __builtin_amdgcn_readfirstlane(a.i0);  // (the divisions left them in VGPRs)
+  a.i1 = __builtin_amdgcn_readfirstlane(a.i1);
   return a;
 }
 
