@@ -481,49 +481,6 @@ void restrict_(psb_ctx *C, const Level<T> &f, const T *e, Level<T> &cL, T omega,
 // ---------------------------------------------------------------------------
 // two stages of a level in one pass (psb_two.h)
 // ---------------------------------------------------------------------------
-// Tile and slab for a level: rows whole where four of them fit a block, else
-// split along k; of the row counts and slab depths the cheapest by
-//   rounds of blocks over the CUs * planes per block * waves on a CU
-// (what the redundant rows and planes cost against CUs without a block;
-// measured at 256^3, FP32: R = 8 and 32 planes, one block per CU, 90 us, R = 8
-// and 16 planes 97, R = 4 and 64 planes 106, R = 10 and 28 planes, 260 blocks,
-// 127).  The registers allow 3 waves per SIMD.
-template <typename T>
-bool two_shape(const psb_ctx *C, const Grid &g, TwoShape &s) {
-  constexpr int V = vmax<T>();
-  if (!C->two || g.nz % V != 0) return false;
-  const int nv = g.nz / V;
-  double best = 0.0;
-  for (const int KO : {nv, 64, 32, 16}) {
-    if (KO > nv || (KO != nv && best > 0.0)) continue;
-    const int KT = KO == nv ? nv : KO + 2, ntk = (nv + KO - 1) / KO;
-    for (int R = 2; (R + 2) * KT <= kTwoThreads; R += 2) {
-      const size_t lds = (size_t)(2 * (R + 4) + 2 * (R + 2) + R) * KT * V;
-      if (lds * sizeof(T) > 150 * 1024) break;
-      const int waves = ((R + 2) * KT + 63) / 64, per_cu = std::max(1, 12 / waves);
-      const long long nt = (long long)((g.ny + R - 1) / R) * ntk;
-      for (int TI = 2; TI < g.nx + 2; TI += 2) {
-        const long long nb = nt * ((g.nx + TI - 1) / TI);
-        const long long rounds = (nb + 256 * per_cu - 1) / (256 * per_cu);
-        const long long act = std::min<long long>(per_cu, (nb + 255) / 256);
-        const double cost = (double)rounds * (TI + 2) * (4 + waves * act);
-        if (nb >= (1 << 30) || (best > 0.0 && cost >= best)) continue;
-        best = cost;
-        s.RT = R + 2;
-        s.KT = KT;
-        s.KO = KO;
-        s.ntj = (g.ny + R - 1) / R;
-        s.ntk = ntk;
-        s.lds = lds;
-        s.TI = TI;
-        s.nblocks = (int)nb;
-        s.threads = waves * 64;
-      }
-    }
-  }
-  return best > 0.0;
-}
-
 // the last pre-sweep of level lv (e to eout; e NULL: from the first sweep omega
 // r / c, formed in the pass) and the restriction to cL in one pass; false where
 // the level does not suit it
@@ -548,8 +505,8 @@ void pre_restrict_m(psb_ctx *C, const Level<T> &lv, DMat<M> A, const T *e, T *eo
 template <typename T>
 bool pre_restrict(psb_ctx *C, const Level<T> &lv, const T *e, T *eout, Level<T> &cL, T omega,
                   T omegaH, DevState *st) {
-  TwoShape s{};
-  if (lv.ae || cL.CI != 2 || cL.CJ != 2 || !two_shape<T>(C, lv.g, s)) return false;
+  const TwoShape &s = lv.two;
+  if (!C->two || lv.ae || cL.CI != 2 || cL.CJ != 2 || s.nblocks == 0) return false;
   if (std::is_same<T, float>::value && !lv.d) return false;
   // four coefficient arrays, r, e in, e out; the coarse cells' c, r and e
   ProbeScope ps(C, PSB_K_RESTRICT, lv.g,
@@ -579,10 +536,9 @@ constexpr int kFirstCells = 1 << 22;
 template <typename T>
 bool first_in_pass(const psb_ctx *C, const Hier<T> &H, int nu1) {
   const Level<T> &lv = H.L[0], &cL = H.L[1];
-  TwoShape s{};
   return nu1 == 2 && lv.g.N >= kFirstCells && !lv.ae &&
          !(std::is_same<T, float>::value && !lv.d) && !tail_at(C, H, 0) && cL.CI == 2 &&
-         cL.CJ == 2 && two_shape<T>(C, lv.g, s);
+         cL.CJ == 2 && C->two && lv.two.nblocks > 0;
 }
 
 // the two post-sweeps of level lv in one pass (e and the correction eH of cL
@@ -605,8 +561,8 @@ void post_two_m(psb_ctx *C, const Level<T> &lv, DMat<M> A, const T *e, T *eout,
 template <typename T, bool RHO>
 bool post_two(psb_ctx *C, const Level<T> &lv, const T *e, T *eout, const Level<T> &cL,
               const T *eH, T cfac, T omega, T zscale, DevState *st, const T *qf) {
-  TwoShape s{};
-  if (lv.ae || !two_shape<T>(C, lv.g, s) || s.nblocks > kMaxBlocks) return false;
+  const TwoShape &s = lv.two;
+  if (!C->two || lv.ae || s.nblocks == 0 || s.nblocks > kMaxBlocks) return false;
   if (std::is_same<T, float>::value && !lv.d) return false;
   // four coefficient arrays, r, e in, e out; the coarse correction, q, the flags
   ProbeScope ps(C, RHO ? PSB_K_SWEEP_LAST : PSB_K_SWEEP_PROL, lv.g,
@@ -942,6 +898,7 @@ void build_hier64(psb_ctx *C) {
   for (int l = 0; l < nl; l++) {
     Level<double> &lv = H.L[l];
     lv.g = make_grid(d[3 * l], d[3 * l + 1], d[3 * l + 2]);
+    lv.two = two_shape<double>(lv.g);
     if (l > 0) {
       lv.CI = d[3 * (l - 1)] / lv.g.nx;
       lv.CJ = d[3 * (l - 1) + 1] / lv.g.ny;
@@ -1032,6 +989,7 @@ void build_hier32(psb_ctx *C) {
     const Level<double> &s = H64.L[l];
     Level<float> &lv = H.L[l];
     lv.g = s.g;
+    lv.two = two_shape<float>(lv.g);
     lv.CI = s.CI; lv.CJ = s.CJ; lv.CK = s.CK;
     lv.aflag = s.aflag;
     const int N = lv.g.N;

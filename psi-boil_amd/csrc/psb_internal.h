@@ -16,6 +16,7 @@
 
 #include "../../include/psb.h"
 #include "psb_kernels.h"
+#include "psb_two.h"
 
 namespace psb {
 namespace host {
@@ -134,6 +135,8 @@ struct Level {
   T *kc = nullptr, *kv = nullptr, *kz = nullptr;
   T *krt = nullptr;  // the second Krylov step's right-hand side (fused kc_r + sweep)
   double *kst = nullptr;
+  // tile of the two-stage passes (two_shape; nblocks 0: one kernel per stage)
+  TwoShape two{};
   // east, north and top couplings of a non-symmetric level (the reference's
   // AC cycle on a 7-array matrix); NULL: symmetric storage (c, w, s, b)
   T *ae = nullptr, *an = nullptr, *at = nullptr;

@@ -41,6 +41,52 @@ struct TwoShape {
   size_t lds;      // elements
 };
 
+// Tile and slab for a level: rows whole where four of them fit a block, else
+// split along k; of the row counts and slab depths the cheapest by
+//   rounds of blocks over the CUs * planes per block * waves on a CU
+// (what the redundant rows and planes cost against CUs without a block;
+// measured at 256^3, FP32: R = 8 and 32 planes, one block per CU, 90 us, R = 8
+// and 16 planes 97, R = 4 and 64 planes 106, R = 10 and 28 planes, 260 blocks,
+// 127).  The registers allow 3 waves per SIMD.  nblocks 0: the rows have no
+// whole vectors.  The search costs 2 to 30 us of the host, so that it is made
+// once per level, and looks at each number of slabs once (at its shallowest
+// depth) and at a row count only where it changes the tiles or the waves.
+template <typename T>
+inline TwoShape two_shape(const Grid &g) {
+  constexpr int V = 16 / (int)sizeof(T);
+  TwoShape s{};
+  if (g.nz % V != 0) return s;
+  const int nv = g.nz / V;
+  double best = 0.0;
+  for (const int KO : {nv, 64, 32, 16}) {
+    if (KO > nv || (KO != nv && best > 0.0)) continue;
+    const int KT = KO == nv ? nv : KO + 2, ntk = (nv + KO - 1) / KO;
+    int waves = 0, ntj = 0;
+    for (int R = 2; (R + 2) * KT <= kTwoThreads; R += 2) {
+      const size_t lds = (size_t)(2 * (R + 4) + 2 * (R + 2) + R) * KT * V;
+      if (lds * sizeof(T) > 150 * 1024) break;
+      if (((R + 2) * KT + 63) / 64 == waves && (g.ny + R - 1) / R == ntj) continue;
+      waves = ((R + 2) * KT + 63) / 64;
+      ntj = (g.ny + R - 1) / R;
+      const int per_cu = 12 / waves > 1 ? 12 / waves : 1;
+      const long long nt = (long long)ntj * ntk;
+      for (int TI = 2, slabs;; TI = ((g.nx + slabs - 2) / (slabs - 1) + 1) & ~1) {
+        slabs = (g.nx + TI - 1) / TI;
+        const long long nb = nt * slabs, cus = (nb + 255) / 256;
+        const long long rounds = (nb + 256 * per_cu - 1) / (256 * per_cu);
+        const long long act = cus < per_cu ? cus : per_cu;
+        const double cost = (double)rounds * (TI + 2) * (4 + waves * act);
+        if (nb < (1 << 30) && !(best > 0.0 && cost >= best)) {
+          best = cost;
+          s = TwoShape{R + 2, KT, KO, ntj, ntk, TI, (int)nb, waves * 64, lds};
+        }
+        if (slabs == 1) break;
+      }
+    }
+  }
+  return s;
+}
+
 // V values at a byte offset from a uniform pointer: the offset of a thread's
 // vector in its plane is constant, the plane's base advances in scalar
 // registers, and a load takes no vector instruction or register for its
