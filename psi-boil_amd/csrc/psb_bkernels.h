@@ -280,7 +280,7 @@ __global__ __launch_bounds__(kBlock) void kb_finalize(int op, const BSeg *fsegs,
   const int sys = blockIdx.x;
   const BFine &F = fine[sys];
   DevState *st = F.st;
-  if (!fin_skip(op, st)) {
+  if (!fin_skip(op, st->done, st->update)) {
     double acc[NR];
     fin_sum<NR>(fsegs[sys].b0, fsegs[sys].nb, partial, acc);
     if (threadIdx.x == 0) fin_apply(op, acc, st, nullptr, nullptr);

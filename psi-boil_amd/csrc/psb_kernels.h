@@ -154,14 +154,14 @@ __device__ inline void krylov_init(DevState *st, double res, double rsq, double 
 }
 
 // steps of a finished loop (or a refresh not pending) do nothing
-__device__ inline bool fin_skip(int op, const DevState *st) {
+__device__ inline bool fin_skip(int op, int done, int update) {
   switch (op) {
     case FIN_PQ: case FIN_XR_DIAG: case FIN_XR_AC: case FIN_RHO: case FIN_RHO_FLEX:
     case FIN_XR_RU:
     case FIN_BI1: case FIN_BI2: case FIN_BI3:
-      return st->done != 0;
+      return done != 0;
     case FIN_RU:
-      return st->done || !st->update;
+      return done || !update;
     default:
       return false;
   }
@@ -188,13 +188,18 @@ __device__ __forceinline__ void fin_rows(int b0, int nblk, const double *partial
   }
 }
 template <int NR>
-__device__ inline void fin_sum(int b0, int nblk, const double *partial, double (&acc)[NR]) {
-  __shared__ double sm[kWaves][NR];
+__device__ __forceinline__ void fin_part(int b0, int nblk, const double *partial,
+                                         double (&acc)[NR]) {
 #pragma unroll
   for (int r = 0; r < NR; r++) acc[r] = 0.0;
   if (nblk <= kBlock) fin_rows<NR, 1>(b0, nblk, partial, acc);
   else if (nblk <= 2 * kBlock) fin_rows<NR, 2>(b0, nblk, partial, acc);
   else fin_rows<NR, 4>(b0, nblk, partial, acc);
+}
+template <int NR>
+__device__ inline void fin_sum(int b0, int nblk, const double *partial, double (&acc)[NR]) {
+  __shared__ double sm[kWaves][NR];
+  fin_part<NR>(b0, nblk, partial, acc);
   block_sum<NR>(acc, sm);
 }
 
@@ -372,42 +377,38 @@ __device__ inline void fin_apply(int op, const double *tot, DevState *st, DevSta
   }
 }
 
-// the scalar step of op on a copy of the state in LDS, which the whole
-// block loads at once beside the partials (the step reads a dozen fields in
-// turn: a round trip to memory each if they were read where they lie).  On
-// return S is in, changed by the step.
-template <int NR>
-__device__ inline void lds_step(int op, int nblk, const double *partial, const DevState *in,
-                                DevState &S, bool record, DevState *st2 = nullptr,
-                                double *out = nullptr) {
-  uint64_t *const sw = reinterpret_cast<uint64_t *>(&S);
-  for (int q = threadIdx.x; q < kStateWords; q += kBlock)
-    sw[q] = reinterpret_cast<const uint64_t *>(in)[q];
-  double tot[NR];
-  fin_sum<NR>(0, nblk, partial, tot);  // its barriers cover S too
-  if (threadIdx.x == 0 && !fin_skip(op, &S)) {
-    double *const hist = S.hist;
-    if (!record) S.hist = nullptr;
-    fin_apply(op, tot, &S, st2, out);
-    S.hist = hist;
-  }
-  __syncthreads();
-}
-
-__device__ inline void put_state(const DevState &S, DevState *out) {
-  const uint64_t *const sw = reinterpret_cast<const uint64_t *>(&S);
-  for (int q = threadIdx.x; q < kStateWords; q += kBlock)
-    reinterpret_cast<uint64_t *>(out)[q] = sw[q];
-}
-
-// one block: st = in after the step (in may be st)
+// One block: st = in after the step of op (in may be st).  The step is taken on
+// a copy of the state in LDS, which the whole block loads at once beside the
+// partials: it reads a dozen fields in turn, a round trip to memory each if they
+// were read where they lie.  A step that does nothing (a loop of fixed length
+// whose solve has stopped launches most of its steps so) ends with those loads:
+// no sums, and no state written where it already lies.
 template <int NR>
 __global__ __launch_bounds__(kBlock) void k_finalize(int op, int nblk, const double *partial,
                                                      const DevState *in, DevState *st,
                                                      DevState *st2, double *out) {
   __shared__ DevState S;
-  lds_step<NR>(op, nblk, partial, in, S, true, st2, out);
-  put_state(S, st);
+  __shared__ double sm[kWaves][NR];
+  // (read as vectors: a scalar load would be waited for with the arguments,
+  // before the partials' loads)
+  int zero = 0;
+  asm("" : "+v"(zero));
+  const int done = in[zero].done, update = in[zero].update;
+  static_assert(kStateWords <= kBlock, "a word per thread");
+  const int t = (int)threadIdx.x;
+  const uint64_t word = reinterpret_cast<const uint64_t *>(in)[min(t, kStateWords - 1)];
+  double tot[NR];
+  fin_part<NR>(0, nblk, partial, tot);
+  if (t < kStateWords) reinterpret_cast<uint64_t *>(&S)[t] = word;
+  const bool skip = __builtin_amdgcn_readfirstlane(fin_skip(op, done, update));
+  if (skip && in == st) return;
+  if (!skip) {
+    block_sum<NR>(tot, sm);  // its barriers cover S too
+    if (t == 0) fin_apply(op, tot, &S, st2, out);
+  }
+  __syncthreads();
+  if (t < kStateWords)
+    reinterpret_cast<uint64_t *>(st)[t] = reinterpret_cast<const uint64_t *>(&S)[t];
 }
 
 // The step in the kernel that uses its result, instead of a one-block launch
