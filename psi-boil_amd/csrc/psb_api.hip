@@ -3090,6 +3090,15 @@ int psb_update_rhs_device(psb_ctx *C, const double *d_u, const double *d_v, cons
   });
 }
 
+// planes per thread of the projection: up to 16, fewer where that leaves the
+// chip idle, and one on planes of less than a wave, whose threads would read
+// pieces of less than a line at once
+static int project_slab(const Grid &g) {
+  int TI = g.sI < 64 ? 1 : 16;
+  while (TI > 1 && (long long)g.sI * ((g.nx + TI - 1) / TI) < 2048LL * kBlock) TI /= 2;
+  return TI;
+}
+
 int psb_project_device(psb_ctx *C, const double *d_rho, const double *d_p, double dt, int mask,
                        double *d_u, double *d_v, double *d_w) {
   if (!C || !d_rho || !d_p || mask < 0 || mask > 7) return PSB_EINVAL;
@@ -3097,13 +3106,11 @@ int psb_project_device(psb_ctx *C, const double *d_rho, const double *d_p, doubl
   if (!C->have_matrix || !C->metrics.dxc) return PSB_ENOTREADY;
   return guarded(C, [&]() {
     const Grid &g = C->g;
-    // slabs of up to 16 planes, fewer where that leaves the chip idle
-    const int ntiles = (g.ny * g.nz + kBlock - 1) / kBlock;
-    int TI = 16;
-    while (TI > 1 && (long long)ntiles * ((g.nx + TI - 1) / TI) < 2048) TI /= 2;
-    hipLaunchKernelGGL(k_project, dim3(ntiles * ((g.nx + TI - 1) / TI)), dim3(kBlock), 0,
-                       C->stream, g, C->metrics, d_rho, C->off_dev, d_p, dt, mask, d_u, d_v, d_w,
-                       TI, ntiles);
+    const int TI = project_slab(g), total = g.sI * ((g.nx + TI - 1) / TI);
+    const auto kernel = C->off_dev ? TI > 1 ? k_project<true, true> : k_project<true, false>
+                                   : TI > 1 ? k_project<false, true> : k_project<false, false>;
+    hipLaunchKernelGGL(kernel, dim3((total + kBlock - 1) / kBlock), dim3(kBlock), 0, C->stream, g,
+                       C->metrics, d_rho, C->off_dev, d_p, dt, mask, d_u, d_v, d_w, TI, total);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(C->stream));
     return (int)PSB_OK;

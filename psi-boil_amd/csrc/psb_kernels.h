@@ -2017,19 +2017,23 @@ static __global__ void k_rhs_center(Grid g, double *b, const uint8_t *off, const
 // 64 B per cell: p, rho, and the three face arrays read and written.
 // A thread walks planes [slab * TI, + TI) at one (j, k): the plane's index is
 // found once, p and rho of the plane below stay in registers, and the next
-// plane's loads are under way while this one's six divisions are computed
-// (201 x 180 x 222: 110 us, 4.7 TB/s, against 130 for one cell at a time; with
-// 8 planes a slab 110, with 32 115 and with 64 133, when blocks are few).
-static __global__ __launch_bounds__(kBlock) void k_project(Grid g, DevMetrics m,
-                                                           const double *rho, const uint8_t *off,
-                                                           const double *p, double dt, int mask,
-                                                           double *u, double *v, double *wv,
-                                                           int TI, int ntiles) {
-  const int slab = (int)blockIdx.x / ntiles, tile = (int)blockIdx.x - slab * ntiles;
-  const int t = tile * kBlock + (int)threadIdx.x, plane = g.ny * g.nz;
-  if (t >= plane) return;
-  int none, j, k;
-  g.ijk(t, none, j, k);
+// plane's loads (dxw and the solid flags among them) are under way while this
+// one's divisions are computed (a call at 256^3 229 us against 272 for one cell at
+// a time, 128^3 with solid cells 40 against 44; slabs of 8, 16, 32, 64 planes at
+// 201 x 180 x 222: 110, 110, 115, 133 us, when blocks are few).  Threads are
+// numbered slab by slab, so that planes smaller than a block leave none idle
+// (50000 x 3 x 5: 24 us, with a block per slab 42); project_slab has the depth.
+// (WALK false: one plane, no loads ahead)
+template <bool OFF, bool WALK>
+__global__ __launch_bounds__(kBlock) void k_project(Grid g, DevMetrics m, const double *rho,
+                                                    const uint8_t *off, const double *p, double dt,
+                                                    int mask, double *u, double *v, double *wv,
+                                                    int TI, int total) {
+  const int id = (int)(blockIdx.x * kBlock + threadIdx.x), plane = g.sI;
+  if (id >= total) return;
+  int slab, j, k;
+  g.ijk(id, slab, j, k);
+  const int t = j * g.nz + k;
   const int i0 = slab * TI, i1 = min(i0 + TI, g.nx);
   const size_t gz = g.nz + 2, gp = (size_t)(g.ny + 2) * gz;
   const double *R = rho + gp + (size_t)(j + 1) * gz + k + 1;  // cell (0, j, k)
@@ -2041,7 +2045,8 @@ static __global__ __launch_bounds__(kBlock) void k_project(Grid g, DevMetrics m,
   const int tS = j > 0 ? t - g.nz : t, tB = k > 0 ? t - 1 : t;
   const size_t rS = j > 0 ? gz : 0, rB = k > 0 ? 1 : 0;
   struct Cell {
-    double p, pS, pB, r, rS, rB, u, v, w;
+    double p, pS, pB, r, rS, rB, u, v, w, dW;
+    uint8_t o, oS, oB;  // solid: the cell, its south and bottom neighbours
   };
   auto load = [&](int i) {
     Cell c;
@@ -2055,35 +2060,43 @@ static __global__ __launch_bounds__(kBlock) void k_project(Grid g, DevMetrics m,
     c.u = fu ? U[(size_t)i * plane] : 0.0;
     c.v = fv ? Vf[i * pv] : 0.0;
     c.w = fw ? Wf[i * pw] : 0.0;
+    c.dW = m.dxw[i];
+    c.o = c.oS = c.oB = 0;
+    if (OFF) {
+      const uint8_t *O = off + (size_t)i * plane;
+      c.o = O[t];
+      c.oS = O[tS];
+      c.oB = O[tB];
+    }
     return c;
   };
   const double dS = m.dys[j], dB = m.dzb[k];
   const int ib = max(i0 - 1, 0);
   double pW = p[(size_t)ib * plane + t], rW = R[(size_t)ib * gp];
+  uint8_t oW = OFF ? off[(size_t)ib * plane + t] : 0;
   Cell c = load(i0);
   for (int i = i0; i < i1; i++) {
     Cell n = c;
-    if (i + 1 < i1) n = load(i + 1);
-    const uint8_t *o = off ? off + (size_t)i * plane : nullptr;
-    const bool fluid = !(o && o[t]);
+    if (WALK && i + 1 < i1) n = load(i + 1);
     if (fu && i > 0) {
       const double rf = 0.5 * (c.r + rW);
-      if (!off) U[(size_t)i * plane] = c.u + (pW - c.p) / rf * dt / m.dxw[i];
-      else if (fluid && !(o - plane)[t])
-        U[(size_t)i * plane] = c.u + (pW - c.p) * dt / rf / m.dxw[i];
+      if (!OFF) U[(size_t)i * plane] = c.u + (pW - c.p) / rf * dt / c.dW;
+      else if (!c.o && !oW) U[(size_t)i * plane] = c.u + (pW - c.p) * dt / rf / c.dW;
     }
     if (fv) {
       const double rf = 0.5 * (c.r + c.rS);
-      if (!off) Vf[i * pv] = c.v + (c.pS - c.p) / rf * dt / dS;
-      else if (fluid && !o[tS]) Vf[i * pv] = c.v + (c.pS - c.p) * dt / rf / dS;
+      if (!OFF) Vf[i * pv] = c.v + (c.pS - c.p) / rf * dt / dS;
+      else if (!c.o && !c.oS) Vf[i * pv] = c.v + (c.pS - c.p) * dt / rf / dS;
     }
     if (fw) {
       const double rf = 0.5 * (c.r + c.rB);
-      if (!off) Wf[i * pw] = c.w + (c.pB - c.p) / rf * dt / dB;
-      else if (fluid && !o[tB]) Wf[i * pw] = c.w + (c.pB - c.p) * dt / rf / dB;
+      if (!OFF) Wf[i * pw] = c.w + (c.pB - c.p) / rf * dt / dB;
+      else if (!c.o && !c.oB) Wf[i * pw] = c.w + (c.pB - c.p) * dt / rf / dB;
     }
+    if (!WALK) break;
     pW = c.p;
     rW = c.r;
+    oW = c.o;
     c = n;
   }
 }
