@@ -541,6 +541,29 @@ bool first_in_pass(const psb_ctx *C, const Hier<T> &H, int nu1) {
          cL.CJ == 2 && C->two && lv.two.nblocks > 0;
 }
 
+// whether the two post-sweeps of a level are faster in one pass.  The pass is a
+// chain of steps, each a barrier and a round trip to memory: on small levels
+// two launches that stream the level once each are as fast or faster.  us a
+// visit saved by the pass in the solve (FP16 copy / FP64):
+//   last sweep with the rho partials: 32^3 -1.9 / -2.0, 48^3 +1.8 / -2.0, 64^3
+//     -1.0 / -4.6, 192 x 32 x 32 -2.7 / -2.7, 72^3 +4.0 / +2.8, 96^3 +2.6 / +4.2,
+//     64 x 64 x 128 -0.9 / -1.2, 128 x 64 x 96 +3.4 / +6.2, 128^3 +3.7 / +9.5
+//   levels of the marching sweeps: 32^3 -1.0 / +0.4, 40^3 0.0 / -0.5, 48^3 -0.7 /
+//     +1.6, 56^3 -1.0 / +1.6, 64^3 -1.4 / +0.1, 64 x 32 x 48 -1.5 / -0.3
+//   below them, one vector per thread in the sweeps: 20^3 -1.8 / -0.9, 16 x 16 x
+//     32 -1.3 / -0.1, 8 x 8 x 128 -2.8 / -2.2, 48 x 8 x 8 -0.9 / -1.3, 96 x 16 x 16
+//     -1.8 / +1.0; two (their grid is a multiple of 8 blocks): 24^3 +2.6 / +2.0,
+//     28^3 +1.6 / +1.6, 24 x 12 x 40 +2.0 / +2.1
+// (The pre-sweep with the restriction gains or ties at all of these.)
+constexpr int kPostTwoCells = 1 << 18;
+template <typename T>
+bool post_two_pays(const Grid &g, bool rho) {
+  if (g.N > kPostTwoCells) return true;
+  if (rho) return false;
+  if (g.N >= kMarchMin) return std::is_same<T, double>::value;
+  return g.N / vmax<T>() > kBlock * nblocks<T>(g);
+}
+
 // the two post-sweeps of level lv in one pass (e and the correction eH of cL
 // to eout); false where the level does not suit it
 template <typename T, bool RHO, typename M, bool FLUX>
@@ -1345,9 +1368,9 @@ T *vcycle(psb_ctx *C, Hier<T> &H, int l, DevState *st, int nu1, int nu2, T omega
   T *zH = kc ? kstep<T>(C, H, l + 1, st, nu1, nu2, omega, cfac)
              : vcycle<T>(C, H, l + 1, st, nu1, nu2, omega, cfac);
   const T cfac_l = T((kc ? 1.0 : (double)cfac) * (cL.scale / lv.scale));
-  if (nu2 == 2) {  // both post-sweeps in one pass where the level suits it
+  const bool rho = l == 0 && rho0;
+  if (nu2 == 2 && post_two_pays<T>(lv.g, rho)) {  // in one pass where the level suits it
     const int out = (cur + 2) % 3;
-    const bool rho = l == 0 && rho0;
     const bool done =
         rho ? post_two<T, true>(C, lv, lv.e[cur], lv.e[out], cL, zH, cfac_l, omega, T(lv.scale),
                                 st, H.qf)
