@@ -175,12 +175,26 @@ BSeg level_seg(const psb_batch *B, int l, int s, long long nwork) {
 // out evenly.  Measured, 96 systems of 32 to 128 cells a side, us, level 0 / 1:
 // 256 threads 162 / 28, 384 (one block to a unit) 214 / 47, 768 214 / 49, 128
 // (rows of 128 cells in blocks of 768) 396 / 27.
+// A launch takes the threads and the LDS of its largest tile for every block, so
+// that one system of long rows would cost all the others their blocks' company:
+// beside systems whose rows fit kBatchTwo threads (small) long rows are split (two
+// of 128^3 and one of 32 x 32 x 256: V-cycle solves 4.86 ms with whole rows, 4.00
+// split, 4.29 with one kernel per stage; 8 of 32^3 and one of 64 x 64 x 384 2.84,
+// 2.44, 2.82).
 constexpr int kBatchTwo = 256;
-void batch_two_shape(const Grid &g, int TI, TwoShape &s) {
+bool batch_rows_fit(int cap, int KT) { return cap / KT - 2 >= 6; }
+void batch_two_shape(const Grid &g, int TI, bool small, TwoShape &s) {
   const int nv = g.nz / 4;
   int KO = nv, KT = nv, cap = kBatchTwo;
-  if ((cap / KT - 2) < 6) cap = kTwoThreads;
-  if ((cap / KT - 2) < 6) {
+  if (!batch_rows_fit(cap, KT)) {
+    if (small) {
+      KO = 16;
+      KT = KO + 2;
+    } else {
+      cap = kTwoThreads;
+    }
+  }
+  if (!batch_rows_fit(cap, KT)) {
     KO = 32;
     KT = KO + 2;
   }
@@ -202,7 +216,10 @@ void batch_two_shape(const Grid &g, int TI, TwoShape &s) {
 // halves x and y (and all or none z).  Depth of the slabs: the rounds of blocks,
 // three to a compute unit and one more that is partly empty, times the steps of
 // one (measured as above, 32 / 16 / 8 / 4 planes: level 0 194 / 162 us, level 1
-// 43 / 28 / 28 / 32)
+// 43 / 28 / 28 / 32).  None where the blocks would be launched with more than two
+// and a half times the threads their tiles have in all: 32 systems of 256 x 8 x 8
+// beside one of 8 x 8 x 256 (3.0 times) 5.91 ms with the pass, 4.94 with one
+// kernel per stage; level 2 of the 96 systems above (2.2 times) no difference.
 void build_two(psb_batch *B, int l) {
   TwoList &W = B->twoL[l];
   const std::vector<BSeg> &who = B->smoothL[l].segs;
@@ -212,13 +229,16 @@ void build_two(psb_batch *B, int l) {
     const BLev<float> &H = B->lev[l + 1][q.sys];
     if (!B->sys[q.sys]->two || !H.sI || !H.sJ || H.sK != sK) return;
   }
+  bool small = false;
+  for (const BSeg &q : who)
+    if (batch_rows_fit(kBatchTwo, B->lev[l][q.sys].g.nz / 4)) small = true;
   long long least = 0;
   int depth = 2;
   for (int TI = 32; TI >= 2; TI /= 2) {
     long long blocks = 0;
     TwoShape s;
     for (const BSeg &q : who) {
-      batch_two_shape(B->lev[l][q.sys].g, TI, s);
+      batch_two_shape(B->lev[l][q.sys].g, TI, small, s);
       blocks += s.nblocks;
     }
     const long long cost = (blocks + 768) * (TI + 3);
@@ -227,14 +247,19 @@ void build_two(psb_batch *B, int l) {
       depth = TI;
     }
   }
-  for (const BSeg &q : who) batch_two_shape(B->lev[l][q.sys].g, depth, B->lev[l][q.sys].two);
-  W.CK = sK ? 2 : 1;
+  long long blocks = 0, used = 0;
   for (const BSeg &q : who) {
-    const TwoShape &s = B->lev[l][q.sys].two;
+    TwoShape &s = B->lev[l][q.sys].two;
+    batch_two_shape(B->lev[l][q.sys].g, depth, small, s);
     W.threads = std::max(W.threads, s.threads);
     W.lds = std::max(W.lds, s.lds * sizeof(float));
-    W.L.segs.push_back(BSeg{q.sys, 0, round8(s.nblocks), 0});
+    blocks += s.nblocks;
+    used += (long long)s.nblocks * s.threads;
   }
+  if (2 * blocks * W.threads > 5 * used) return;
+  W.CK = sK ? 2 : 1;
+  for (const BSeg &q : who)
+    W.L.segs.push_back(BSeg{q.sys, 0, round8(B->lev[l][q.sys].two.nblocks), 0});
   upload_list(B, W.L);
 }
 
