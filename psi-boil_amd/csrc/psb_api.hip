@@ -2269,7 +2269,7 @@ void build_ref(psb_ctx *C) {
   if (nl < 2) throw std::invalid_argument("grid too small for the AC cycle");
   H.L.assign(nl, Level<double>());
   H.M.assign(nl, Metric{nullptr, nullptr, nullptr});
-  H.K.assign(nl, std::vector<double *>(5, nullptr));
+  H.K.assign(nl, {});
   std::vector<double> hx = C->gdx, hy = C->gdy, hz = C->gdz;
   if (hx.empty()) {
     hx.assign(C->g.nx, 1.0);
@@ -2323,7 +2323,8 @@ void build_ref(psb_ctx *C) {
     lv.r = C->harena.alloc<double>(N);     // f of this level
     lv.e[0] = C->harena.alloc<double>(N);  // phi
     if (l == 0) lv.e[1] = C->harena.alloc<double>(N);  // phi of the previous cycle
-    for (int q = 0; q < 5; q++) H.K[l][q] = C->harena.alloc<double>(N);
+    H.K[l].resize(cg_di_fold(C, lv.g, true) ? 5 : 4);  // z where the level's solve folds
+    for (double *&v : H.K[l]) v = C->harena.alloc<double>(N);
   }
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(stream));
@@ -2344,9 +2345,9 @@ void ref_cg(psb_ctx *C, int l, int maxit, double res_rat, double res_tol, double
                      scale, (double)g.N, stalecount);
   zero(C, p0, g.N);
   zero(C, p1, g.N);
-  double *const p[2] = {p0, p1}, *const qz[2] = {q, H.K[l][4]};
-  start<double, SYM, 0>(C, g, lv.mat(), lv.r, lv.e[0], r, cg_di_fold(C, g, true) ? q : nullptr, 0.0, st,
-                        &H.M[l]);
+  const bool fold = cg_di_fold(C, g, true);
+  double *const p[2] = {p0, p1}, *const qz[2] = {q, fold ? H.K[l][4] : nullptr};
+  start<double, SYM, 0>(C, g, lv.mat(), lv.r, lv.e[0], r, fold ? q : nullptr, 0.0, st, &H.M[l]);
   cg_di_run<SYM>(C, g, lv.mat(), r, p, qz, lv.e[0], st, C->st64b, maxit, &H.M[l], verdict);
 }
 
@@ -2355,7 +2356,7 @@ void ref_cg(psb_ctx *C, int l, int maxit, double res_rat, double res_tol, double
 // equation's own Krylov solver (additive_cycle_functions.cpp:89-107), which
 // for the non-symmetric equations is BiCGS.  The kernels and scalar steps
 // of the single-level BiCGS solve (solve_bicgs_diag) on the level's arrays;
-// phi is improved in place.  Work vectors: the CG's five and three more
+// phi is improved in place.  Work vectors: the CG's and more, eight in all
 // (ref_bicgs_buffers, before any capture).
 void ref_bicgs_buffers(psb_ctx *C) {
   RefHier &H = C->href;

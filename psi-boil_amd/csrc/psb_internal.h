@@ -192,7 +192,8 @@ constexpr size_t kGraphCacheMax = 12;
 
 // the reference's AC cycle: its own levels (smallest-prime-factor
 // coarsening), each with phi (e[0]), the right-hand side f (r) and the
-// work vectors of that level's CG (r, p0, p1, q, z); level 0's e[1] holds the
+// work vectors of that level's CG (r, p0, p1, q, and z where it folds its scalar
+// steps); level 0's e[1] holds the
 // previous cycle's phi for the divergence restore
 struct RefHier {
   std::vector<Level<double>> L;
