@@ -870,16 +870,35 @@ std::vector<double> dense_inv(int nx, int ny, int nz, const std::vector<double> 
 }
 
 // dense_pinv's G of level cl by the kernels of psb_dense.h, where the band fits
-// them; false elsewhere (and for 7 arrays)
+// them; false elsewhere (and for 7 arrays).  The factor and the inverse's columns
+// are scratch: the sweeps' vectors of the finest level hold them where they are
+// long enough (no solve of a hierarchy that is being built uses them), else a
+// block of its own, which goes back here.
 bool device_pinv(psb_ctx *C, const Level<double> &cl, double *G) {
   const Grid &g = cl.g;
   const int m = g.N, bw = g.nx > 1 ? g.ny * g.nz : (g.ny > 1 ? g.nz : 1), n = bw + 1;
   if (!C->dense || cl.ae || bw > kBandMax || m > kBandMaxCells) return false;
-  Arena &ar = C->harena;
-  BandArgs A{g.nx, g.ny, g.nz, bw, cl.c, cl.w, cl.s, cl.b, cl.aflag,
-             ar.alloc<double>((size_t)m * n), ar.alloc<double>((size_t)m * n)};
-  double *Bt = ar.alloc<double>((size_t)m * m), *cm = ar.alloc<double>(m),
-         *rm = ar.alloc<double>(m + 1);
+  const size_t mm = (size_t)m * m, mn = (size_t)m * n, sums = 2 * (size_t)m + 1;
+  const Level<double> &f = C->h64.L[0];
+  struct Block {
+    void *p = nullptr;
+    ~Block() {
+      if (p) (void)hipFree(p);
+    }
+  } own;
+  double *Bt = f.e[0], *Lc = f.e[1], *Lr = f.e[2];
+  if (mm > (size_t)f.g.N || mn + sums > (size_t)f.g.N) {
+    if (hipMalloc(&own.p, (mm + 2 * mn + sums) * sizeof(double)) != hipSuccess) {
+      (void)hipGetLastError();
+      own.p = nullptr;
+      return false;  // the host forms it
+    }
+    Bt = static_cast<double *>(own.p);
+    Lc = Bt + mm;
+    Lr = Lc + mn;
+  }
+  double *cm = Lr + mn, *rm = cm + m;
+  BandArgs A{g.nx, g.ny, g.nz, bw, cl.c, cl.w, cl.s, cl.b, cl.aflag, Lc, Lr};
   auto chol = [&](auto u) {
     hipLaunchKernelGGL((k_band_chol<decltype(u)::value>), dim3(1), dim3(kBandThreads),
                        (size_t)n * (n + 1) / 2 * sizeof(double), C->stream, A);
@@ -906,6 +925,7 @@ bool device_pinv(psb_ctx *C, const Level<double> &cl, double *G) {
                        rm + m, G);
   }
   HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(C->stream));
   return true;
 }
 
@@ -960,7 +980,6 @@ void build_hier64(psb_ctx *C) {
   H.m = m;
   H.G = C->harena.alloc<double>((size_t)m * m);
   if (device_pinv(C, cl, H.G)) {
-    HIPCHK(hipStreamSynchronize(stream));
     H.built = true;
     return;
   }

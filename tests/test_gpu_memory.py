@@ -1,7 +1,8 @@
 """Device memory a context holds after a solve: the AC cycle's levels keep the
-fifth vector of their CG only where the folded steps read it.  Compared with a
-context that does without (PSB_NO_FOLD set); the runtime hands memory out in
-pieces of up to 2 MB."""
+fifth vector of their CG only where the folded steps read it, and the dense
+operator of the coarsest level keeps none of the arrays it was formed in.
+Compared with a context that does without (PSB_NO_FOLD, PSB_NO_DENSE set); the
+runtime hands memory out in pieces of up to 2 MB."""
 import ctypes
 import os
 
@@ -44,6 +45,10 @@ def cycle(s, b):
     s.ac_vcycle(np.zeros(b.size), b, max_cycles=1)
 
 
+def solve(s, b):
+    s.solve(np.zeros(b.size), b, precond=psb.PSB_PREC_AC, max_iter=4)
+
+
 @pytest.mark.parametrize("shape, folds", [((128, 128, 128), False), ((96, 96, 96), True)])
 def test_cycle_keeps_the_fifth_vector_where_it_folds(shape, folds):
     held(shape, None, cycle)  # (the library's own first allocations)
@@ -53,3 +58,9 @@ def test_cycle_keeps_the_fifth_vector_where_it_folds(shape, folds):
     if folds:
         assert extra >= vector - PIECE
     assert extra <= (vector if folds else 0) + below + PIECE
+
+
+@pytest.mark.parametrize("shape", [(48, 48, 48), (64, 64, 64), (128, 128, 128)])
+def test_dense_operator_keeps_no_scratch(shape):
+    held(shape, None, solve)
+    assert held(shape, None, solve) <= held(shape, "PSB_NO_DENSE", solve) + PIECE
