@@ -236,18 +236,35 @@ void cg_xr(psb_ctx *C, const Grid &g, const T *c, const T *p, const T *q, T *x, 
 // of four, the state handed from st to st2 and back; the last iteration's step
 // ends in st (unless `last` is false: nobody asks for it).  On larger grids only
 // alpha is folded (fold_pq).
-// The line: every block reads every partial, which grows with the blocks squared
-// and at some thousand of them costs what the two launches cost.  us an
-// iteration, folded / not, two-wide cells: 64^3 11.3 / 13.3, 80^3 20.3 / 21.6,
-// 96 x 72 x 72 21.5 / 22.0, 88 x 84 x 84 26.3 / 26.0, 96^3 30.6 / 29.3, 156 x 41 x
-// 146 31.7 / 30.7; scalar cells (odd nz): 57 x 45 x 39 10.9 / 13.1, 50 x 50 x 59
-// 15.9 / 14.8, 80 x 80 x 79 36.2 / 25.8.  The reference's cycle runs its levels'
-// solves for a fixed number of iterations, most of them after they have stopped,
-// where only the launches count: two cycles of 96^3 8.3 ms folded up to 2^20
-// two-wide cells, 8.9 up to 2^19 (12.5 not folded).
+// The line: every block reads every partial of the kernel before, so that the
+// fold's cost grows with the product of the two kernels' blocks and at some
+// 540 000 is what the two launches cost.  us an iteration of 40 iterations' solves,
+// folded / not, at the product in thousands: two-wide cells 64^3 (262) 15.5 / 17.3, 96 x 72 x 72 (511)
+// 26.0 / 26.8, 80^3 (520) 24.8 / 26.2, 88 x 76 x 76 (524) 26.1 / 27.1, 1500 x 16 x
+// 16 (558) 24.8 / 23.8, 96 x 64 x 64 (590) 20.9 / 20.1, 112 x 64 x 64 (803) 23.3 /
+// 21.7, 128 x 64 x 64 (1049) 24.5 / 22.6; scalar cells (odd nz): 57 x 45 x 39 10.9 /
+// 13.1, 50 x 50 x 59 15.9 / 14.8, 80 x 80 x 79 36.2 / 25.8.
+// The reference's cycle runs its levels' solves for a fixed number of iterations,
+// most of them after they have stopped, where only the launches count.  Two
+// cycles, ms, finest level folded / not, the coarser ones folded: 128 x 64 x 64
+// 7.13 / 7.14, 96^3 8.21 / 8.15, 100^3 7.68 / 7.67, 104 x 100 x 100 7.67 / 7.91,
+// 60 x 120 x 140 8.56 / 8.74, 128 x 88 x 92 9.08 / 9.02, 128 x 128 x 64 (2^20 cells)
+// 8.46 / 8.24; no level folded 8.7, 9.9, 10.0, 9.3, 10.2, 12.4, 9.8; scalar cells
+// 81 x 45 x 45 5.12 / 5.16, 75 x 65 x 45 5.69 / 5.11, 81 x 63 x 45 5.43 / 5.51, 80 x
+// 80 x 81 8.02 / 7.40, 96 x 90 x 105 10.5 / 8.8.
 constexpr int kFoldCells = 1 << 20;
+constexpr int kFoldBlocks = 1 << 19;
+// the p/q step's blocks: the marching kernel's tiles and slabs, else spans
+template <int V>
+MarchShape cg_di_shape(const Grid &g) {
+  MarchShape m{0, 0, 0};
+  if (V > 1 && g.N >= kMarchMin && march_ok<V>(g, m)) return m;
+  return MarchShape{0, 0, nblocks<double>(g)};
+}
 bool cg_di_fold(const psb_ctx *C, const Grid &g, bool cycle = false) {
-  return C->fold && g.N <= (!vec_ok<double>(g) ? 1 << 17 : cycle ? kFoldCells : 1 << 19);
+  if (!C->fold || g.N > kFoldCells) return false;
+  if (!vec_ok<double>(g)) return g.N <= 1 << 17;
+  return cycle || cg_di_shape<vmax<double>()>(g).nblocks * nblocks<double>(g) <= kFoldBlocks;
 }
 // q: two arrays with the fold (z of the iteration before is read from one,
 // q[0] at the start, while A p goes to the other); n even unless it ends there
@@ -267,8 +284,7 @@ void cg_di_run(psb_ctx *C, const Grid &g, DMat<double> A, double *r, double *con
       const Fold f{it > 0 ? nxr : 0, C->work.partial, nxt};
       with_v<double>(g, [&](auto vt) {
         constexpr int V = decltype(vt)::value;
-        MarchShape m{0, 0, nxr};
-        if (!(V > 1 && g.N >= kMarchMin && march_ok<V>(g, m))) m = MarchShape{0, 0, nxr};
+        const MarchShape m = cg_di_shape<V>(g);
         npq = m.nblocks;
         hipLaunchKernelGGL((k_cg_pq_di<V, SYM>), dim3(npq), dim3(kBlock), 0, C->stream, g, A,
                            q[it & 1], pold, pnew, q[(it & 1) ^ 1], cur, f, pq_work(C), m.TI,
