@@ -232,6 +232,10 @@ static __global__ __launch_bounds__(kBlock) void k_band_turn(int m, const double
 // additions are then whole numbers and can be taken in any order.  A pass takes
 // 8192 entries up to the first one that is a tie or leaves the interval, adds
 // that one to the sum in floating point, and the next pass goes on behind it.
+// While there is no such interval yet (the sum is 0 through the rows of solid
+// cells before the first active one) a pass skips zeros, which leave the sum as
+// it is, and adds up to 64 entries one by one: 48^3 with its first half solid,
+// a new matrix in 7.1 ms where 64 zeros at a time took 29.5.
 // Measured: 0.27 ms for the 2^18 entries of 8^3 cells, 1.7 ms for the 3.0 M of
 // 12^3 (one after another: 4 ns each).
 constexpr int kTotalPer = 8;
@@ -252,16 +256,29 @@ static __global__ __launch_bounds__(1024) void k_band_total(long long n, const d
     const double s = s_sum;
     if (pos >= n) break;
     if (t == 0) s_bad = 1024 * kTotalPer;
+    double b[kTotalPer];
+#pragma unroll
+    for (int q = 0; q < kTotalPer; q++) {
+      const long long at = pos + t * kTotalPer + q;
+      b[q] = at < n ? B[at] : 0.0;
+    }
     // the first entries, and a sum that is not a normal positive number: singly
     if (pos < 64 || !(s >= 1e-290 && s <= 1e290)) {
-      const int some = (int)min((long long)64, n - pos);
-      if (t < some) head[t] = B[pos + t];
+      int first = 1024 * kTotalPer;
+#pragma unroll
+      for (int q = kTotalPer - 1; q >= 0; q--) first = b[q] != 0.0 ? t * kTotalPer + q : first;
+      __syncthreads();
+      if (first < 1024 * kTotalPer) atomicMin(&s_bad, first);
+      __syncthreads();
+      const long long from = pos + s_bad;
+      const int some = s_bad < 1024 * kTotalPer ? (int)min((long long)64, n - from) : 0;
+      if (t < some) head[t] = B[from + t];
       __syncthreads();
       if (t == 0) {
         double v = s;
         for (int q = 0; q < some; q++) v += head[q];
         s_sum = v;
-        s_pos = pos + some;
+        s_pos = from + some;
       }
       __syncthreads();
       continue;
@@ -269,14 +286,8 @@ static __global__ __launch_bounds__(1024) void k_band_total(long long n, const d
     const int e = (int)(__double_as_longlong(s) >> 52) - 1023;  // s in [2^e, 2^(e + 1))
     const double up = __longlong_as_double((long long)(52 - e + 1023) << 52);
     const double u = __longlong_as_double((long long)(e - 52 + 1023) << 52);
-    double b[kTotalPer];
     long long mine = 0;
     int bad = 1024 * kTotalPer;  // the first entry of this thread that cannot be a whole number
-#pragma unroll
-    for (int q = 0; q < kTotalPer; q++) {
-      const long long at = pos + t * kTotalPer + q;
-      b[q] = at < n ? B[at] : 0.0;
-    }
 #pragma unroll
     for (int q = kTotalPer - 1; q >= 0; q--) {
       const double x = b[q] * up, r = rint(x);
