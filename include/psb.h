@@ -133,9 +133,10 @@ typedef struct {
                             operator on level 0 (its q = A p reads 8 instead
                             of 16 B per cell; the FP64 reliable updates
                             still measure the true residual)                */
-  int ac_fuse;           /* accepted and without effect: the two post-sweeps
-                            of a level run in one pass wherever its shape
-                            allows                                         */
+  int ac_fuse;           /* PSB_MIXED: 1 runs the two post-sweeps of a level
+                            in one pass wherever its shape allows; 0
+                            (default) only on the levels where that is
+                            faster (same z)                                */
   int ac_kcycle;         /* K-cycle levels, bit l for level l (level 1 is the
                             first coarse level; bit 0 must be 0): there the
                             coarse correction is two flexible-CG steps

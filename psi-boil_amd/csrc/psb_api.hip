@@ -1404,7 +1404,8 @@ T *vcycle(psb_ctx *C, Hier<T> &H, int l, DevState *st, int nu1, int nu2, T omega
              : vcycle<T>(C, H, l + 1, st, nu1, nu2, omega, cfac);
   const T cfac_l = T((kc ? 1.0 : (double)cfac) * (cL.scale / lv.scale));
   const bool rho = l == 0 && rho0;
-  if (nu2 == 2 && post_two_pays<T>(lv.g, rho)) {  // in one pass where the level suits it
+  const bool fuse = C->fuse && std::is_same<T, float>::value;
+  if (nu2 == 2 && (fuse || post_two_pays<T>(lv.g, rho))) {  // in one pass
     const int out = (cur + 2) % 3;
     const bool done =
         rho ? post_two<T, true>(C, lv, lv.e[cur], lv.e[out], cL, zH, cfac_l, omega, T(lv.scale),
@@ -1882,6 +1883,7 @@ GKey solve_key(const psb_ctx *C, const psb_stop *p, int body, const void *x, con
   k.nu1 = p->ac_pre;
   k.nu2 = p->ac_post;
   k.kmask = C->kmask;
+  k.fuse = C->fuse;
   k.cg16 = C->cg_half;
   k.half = body == 0 || body >= 3 ? 0 : (C->h32.L.empty() ? 0 : C->h32.L[0].use16);
   k.flex = C->flex;
@@ -2742,6 +2744,7 @@ int solve_device(psb_ctx *C, double *x, const double *b, const psb_stop *p, psb_
         return PSB_EINVAL;
       ensure_rule(C, p->ac_coarsen);
       C->cg_half = false;
+      C->fuse = false;
       C->kmask = 0;
       C->flex = false;
       C->ac_omega = p->ac_omega;
@@ -2760,6 +2763,7 @@ int solve_device(psb_ctx *C, double *x, const double *b, const psb_stop *p, psb_
     // settings of this solve, read while its graph is captured (the graph
     // cache keys on them: no setting change drops a graph)
     C->cg_half = p->precision == PSB_MIXED && p->ac_store == 2;
+    C->fuse = p->ac_fuse != 0;
     C->kmask = p->ac_kcycle;
     C->flex_req = p->ac_flexible;  // resolved against the hierarchy (set_flex)
     C->ac_omega = p->ac_omega;

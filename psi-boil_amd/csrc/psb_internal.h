@@ -173,18 +173,17 @@ struct Graph {
 };
 
 // Everything a captured AC-preconditioned solve bakes into its graph: the
-// kernels chosen (K-cycle levels, FP16 copies, the CG operator's storage,
-// flexible beta), the scalars passed by value (omega, coarse factor) and the
-// caller arrays.  Solves with equal keys replay one
-// graph; a solve with other settings captures its own beside it, so that
+// kernels chosen (K-cycle levels, one-pass post-sweeps, FP16 copies, the CG
+// operator's storage, flexible beta), the scalars passed by value (omega, coarse
+// factor) and the caller arrays.  Solves with equal keys replay one graph; a solve with other settings captures its own beside it, so that
 // switching settings back and forth never destroys a graph in use.
 struct GKey {
   int body = 0;  // 0 FP64 AC-PCG, 1 FP32 inner solve of the refinement, 2 reliable updates
-  int chunk = 0, nu1 = 0, nu2 = 0, kmask = 0, cg16 = 0, half = 0, flex = 0;
+  int chunk = 0, nu1 = 0, nu2 = 0, kmask = 0, fuse = 0, cg16 = 0, half = 0, flex = 0;
   double omega = 0.0, cfac = 0.0;
   const void *px = nullptr, *pb = nullptr;
   auto tie() const {
-    return std::tie(body, chunk, nu1, nu2, kmask, cg16, half, flex, omega, cfac, px, pb);
+    return std::tie(body, chunk, nu1, nu2, kmask, fuse, cg16, half, flex, omega, cfac, px, pb);
   }
   bool operator<(const GKey &o) const { return tie() < o.tie(); }
 };
@@ -259,6 +258,7 @@ struct psb_ctx {
   int coarse_min = 8;  // coarsening halves a direction while it stays >= this
   int coarse_rule = 0; // 0 all directions at once, 1 x and y before z
   // settings of the running AC solve, read while its graph is captured
+  bool fuse = false;        // FP32 post-sweeps in one pass on every level that suits it
   bool cg_half = false;     // the FP32 CG operator reads the level-0 FP16 copy too
   int kmask = 0;            // K-cycle levels (bit l: level l) of the AC hierarchies
   bool flex = false;        // flexible (Polak-Ribiere) beta in the outer CG
