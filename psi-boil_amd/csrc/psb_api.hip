@@ -239,11 +239,11 @@ void cg_xr(psb_ctx *C, const Grid &g, const T *c, const T *p, const T *q, T *x, 
 // The line: every block reads every partial of the kernel before, so that the
 // fold's cost grows with the product of the two kernels' blocks and at some
 // 540 000 is what the two launches cost.  us an iteration of 40 iterations' solves,
-// folded / not, at the product in thousands: two-wide cells 64^3 (262) 15.5 / 17.3, 96 x 72 x 72 (511)
-// 26.0 / 26.8, 80^3 (520) 24.8 / 26.2, 88 x 76 x 76 (524) 26.1 / 27.1, 1500 x 16 x
-// 16 (558) 24.8 / 23.8, 96 x 64 x 64 (590) 20.9 / 20.1, 112 x 64 x 64 (803) 23.3 /
-// 21.7, 128 x 64 x 64 (1049) 24.5 / 22.6; scalar cells (odd nz): 57 x 45 x 39 10.9 /
-// 13.1, 50 x 50 x 59 15.9 / 14.8, 80 x 80 x 79 36.2 / 25.8.
+// folded / not, at the product in thousands: two-wide cells 64^3 (262) 15.5 / 17.3,
+// 96 x 72 x 72 (511) 26.0 / 26.8, 80^3 (520) 24.8 / 26.2, 88 x 76 x 76 (524) 26.1 /
+// 27.1, 1500 x 16 x 16 (558) 24.8 / 23.8, 96 x 64 x 64 (590) 20.9 / 20.1, 112 x 64 x
+// 64 (803) 23.3 / 21.7, 128 x 64 x 64 (1049) 24.5 / 22.6; scalar cells (odd nz) 57 x
+// 45 x 39 10.9 / 13.1, 50 x 50 x 59 15.9 / 14.8, 80 x 80 x 79 36.2 / 25.8.
 // The reference's cycle runs its levels' solves for a fixed number of iterations,
 // most of them after they have stopped, where only the launches count.  Two
 // cycles, ms, finest level folded / not, the coarser ones folded: 128 x 64 x 64

@@ -26,8 +26,13 @@ struct Metric {
   }
 };
 
+// the reductions' partial sums: kMaxBlocks * kMaxPartials doubles, a block's
+// together.  Most kernels leave theirs at the start (up to kRhoParts = 6 a block);
+// the CG's p.q begin at 6 * kMaxBlocks (pq_work), and a folded BiCGS iteration has
+// s.s, t.s and t.t at 0, the x/r step's three at 3 * kMaxBlocks, r~.v at 6 *
+// kMaxBlocks.
 struct Work {
-  double *partial;  // kMaxBlocks * 4 doubles
+  double *partial;
 };
 
 // contiguous run of V-vectors per block of the span; P, i, j, k of the
@@ -55,7 +60,8 @@ struct Work {
 // ---------------------------------------------------------------------------
 // pass 2 of the reductions: the partials of the kernel before it summed in a
 // fixed order and the scalar step applied, by one block (k_finalize) or by
-// every block of the kernel that needs the result (fold_step, fold_pq)
+// every block of the kernel that needs the result (fold_xr_diag, fold_pq,
+// fold_bi1 .. fold_bi3)
 // ---------------------------------------------------------------------------
 enum FinOp {
   FIN_START_DIAG, FIN_START_AC, FIN_START_BICGS, FIN_PQ, FIN_XR_DIAG, FIN_XR_AC, FIN_RHO,

@@ -63,9 +63,14 @@ struct TailArgs {
 // a / c by its correctly rounded reciprocal rc, as the division rounds it:
 // the product is within two units in the last place, each step's remainder is
 // exact, so the first leaves a faithful quotient and the second the rounded one
-// (P. Markstein, IBM J. Res. Dev. 34 (1990) 111-119).  Five instructions where
-// the division takes eleven (FP32) or more; the sweeps divide by one diagonal
-// over and over.
+// (P. Markstein, IBM J. Res. Dev. 34 (1990) 111-119).  That holds while c, rc, the
+// quotient and the remainder are normal numbers: numerators below some 1e-31
+// (FP32; FP64 1e-291) can round their last bit the other way, an infinite one gives
+// NaN where the division gives infinity.  (The preconditioner's values there have
+// lost their digits or the solve has ended: solves with the right-hand side scaled
+// by 1e-300 to 1e300 are those of the separate kernels, NaN for NaN.)  Five
+// instructions where the division takes eleven (FP32) or more; the sweeps divide by
+// one diagonal over and over.
 __device__ __forceinline__ float div_by(float a, float c, float rc) {
   float q = a * rc;
   q = __builtin_fmaf(__builtin_fmaf(-c, q, a), rc, q);

@@ -16,13 +16,19 @@
 //     the others may hold anything.
 //   * Matrix, right-hand side and operand of the next plane are loaded a plane
 //     ahead; a plane's w couplings are the plane before's e.
-// What bounds it: at 256^3 (FP16 copy) the first pair takes 386 MB of HBM
-// traffic (1.07 of what it must move) at 4.4 TB/s with the vector units half
-// busy.  Measured, us, one pass against two kernels:
-//   first pair, FP16 copy: 256^3 87 / 78 + 67, 128^3 18 / 11.5 + 9.3, 32^3 7.1 / 4.5 + 5.5
-//   first pair, FP64:      256^3 216 / 399, 128^3 31 / 25 + 21, 32^3 6.7 / 3.9 + 4.9
-//   post-sweeps, FP16 copy: 256^3 100 / 76 + 81, 128^3 18.6 / 11.5 + 11.7, 32^3 8.2 / 4.5 + 4.7
-//   post-sweeps, FP64:      256^3 278 / 195 + 214, 128^3 25 / 25 + 21, 32^3 6.4 / 4.6 + 4.6
+// What bounds it: at 256^3 (FP16 copy) the first pair, its operand formed from r
+// and c (TwoFirst), takes 385 MB of HBM traffic (1.07 of what it must move) in 99
+// us, 3.9 TB/s with the vector units half busy; the post-sweeps 436 MB (1.06) in
+// 102 us, 4.3 TB/s.  Measured in traced solves, us, one pass against two kernels:
+//   first pair, FP16 copy: 256^3 99 / 78 + 67 (with the first sweep stored, 24 us
+//     more in the x/r step: 87), 128^3 19.7 / 11.5 + 9.3, 64^3 8.8, 32^3 8.0 / 4.5 + 5.5
+//   first pair, FP64:      256^3 217 / 399, 128^3 30 / 25 + 21, 64^3 9.9, 32^3 7.1 / 3.9 + 4.9
+//   post-sweeps, FP16 copy: 256^3 102 / 76 + 81, 128^3 19.0 / 11.5 + 11.7, 64^3 8.6 /
+//     4.8 + 4.7, 32^3 8.2 / 4.5 + 4.7
+//   post-sweeps, FP64:      256^3 278 / 195 + 214, 128^3 26 / 25 + 21, 64^3 8.9, 32^3
+//     6.7 / 4.6 + 4.6
+// In untraced solves small levels gain less than these figures say, or lose:
+// post_two_pays (psb_api.hip) has what a visit gains there and where the line is.
 // The arithmetic is the separate kernels' (gather_c), so that the results are
 // bit-identical; only the rho partials are summed over other blocks.
 #pragma once
