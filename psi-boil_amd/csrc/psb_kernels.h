@@ -194,18 +194,13 @@ __device__ __forceinline__ void fin_rows(int b0, int nblk, const double *partial
   }
 }
 template <int NR>
-__device__ __forceinline__ void fin_part(int b0, int nblk, const double *partial,
-                                         double (&acc)[NR]) {
+__device__ inline void fin_sum(int b0, int nblk, const double *partial, double (&acc)[NR]) {
+  __shared__ double sm[kWaves][NR];
 #pragma unroll
   for (int r = 0; r < NR; r++) acc[r] = 0.0;
   if (nblk <= kBlock) fin_rows<NR, 1>(b0, nblk, partial, acc);
   else if (nblk <= 2 * kBlock) fin_rows<NR, 2>(b0, nblk, partial, acc);
   else fin_rows<NR, 4>(b0, nblk, partial, acc);
-}
-template <int NR>
-__device__ inline void fin_sum(int b0, int nblk, const double *partial, double (&acc)[NR]) {
-  __shared__ double sm[kWaves][NR];
-  fin_part<NR>(b0, nblk, partial, acc);
   block_sum<NR>(acc, sm);
 }
 
@@ -403,8 +398,13 @@ __global__ __launch_bounds__(kBlock) void k_finalize(int op, int nblk, const dou
   static_assert(kStateWords <= kBlock, "a word per thread");
   const int t = (int)threadIdx.x;
   const uint64_t word = reinterpret_cast<const uint64_t *>(in)[min(t, kStateWords - 1)];
+  // (fin_sum's rows; its sums below, once the step is known to be taken)
   double tot[NR];
-  fin_part<NR>(0, nblk, partial, tot);
+#pragma unroll
+  for (int r = 0; r < NR; r++) tot[r] = 0.0;
+  if (nblk <= kBlock) fin_rows<NR, 1>(0, nblk, partial, tot);
+  else if (nblk <= 2 * kBlock) fin_rows<NR, 2>(0, nblk, partial, tot);
+  else fin_rows<NR, 4>(0, nblk, partial, tot);
   if (t < kStateWords) reinterpret_cast<uint64_t *>(&S)[t] = word;
   const bool skip = __builtin_amdgcn_readfirstlane(fin_skip(op, done, update));
   if (skip && in == st) return;
